@@ -648,6 +648,32 @@ int pdk_scatter_paged_layerwise(const pdk_scatter_req* reqs, int n_reqs,
                                 const uintptr_t* wait_events,
                                 uintptr_t stream);
 
+/* ---- prefill -------------------------------------------------------------------
+ * The non-GEMM part of one prompt's prefill (engines/prefill_full.py:337-388),
+ * head_dim 128. table [T][half] (cos, sin) fp32 pairs of t * inv_freq[i]. */
+int pdk_rope_table(const float* inv_freq, int T, int half, float* table,
+                   uintptr_t stream);
+
+/* Elements of each of the two operand buffers kt and vt below. */
+int64_t pdk_prefill_kv_tile_elems(int T, int n_kv_heads);
+
+/* qkv [T][(Hq + 2 Hkv) * 128] bf16, contiguous: q is rotated in place, the
+ * rotated k and the v go to k_out and v_out ([T] rows of [Hkv][128], the given
+ * token strides in elements, multiples of 8) and, as pdk_prefill_attn reads
+ * them, to kt and vt. table is pdk_rope_table's with half = 64. */
+int pdk_prefill_rope_kv(uint16_t* qkv, const float* table, int T, int n_q_heads,
+                        int n_kv_heads, int head_dim, uint16_t* k_out,
+                        int64_t k_tok_stride, uint16_t* v_out,
+                        int64_t v_tok_stride, uint16_t* kt, uint16_t* vt,
+                        uintptr_t stream);
+
+/* Causal GQA attention of the prompt: out [T][Hq][128] bf16 from q (rows of
+ * q_tok_stride elements, Hq * 128 of them used) and pdk_prefill_rope_kv's kt
+ * and vt. Query head h reads KV head h / (Hq / Hkv). Weights stay fp32. */
+int pdk_prefill_attn(const uint16_t* q, int64_t q_tok_stride, const uint16_t* kt,
+                     const uint16_t* vt, int T, int n_q_heads, int n_kv_heads,
+                     int head_dim, float scale, uint16_t* out, uintptr_t stream);
+
 /* ---- streams and events ------------------------------------------------------
  * Fences for the side-stream staging and for wait_for_save()
  * (connector/rngd_kv.py:129-131), which becomes a real barrier once saves

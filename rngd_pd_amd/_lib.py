@@ -129,6 +129,10 @@ SIGNATURES = {
                                      ctypes.c_float, _P, _SZ, _P, _I, _U]),
     "pdk_row_ssq": (_I, [_P, _I, _I, _P, _U]),
     "pdk_embed_ssq": (_I, [_P, _I64, _P, _I, _I, _I, _P, _P, _U]),
+    "pdk_rope_table": (_I, [_P, _I, _I, _P, _U]),
+    "pdk_prefill_kv_tile_elems": (_I64, [_I, _I]),
+    "pdk_prefill_rope_kv": (_I, [_P, _P, _I, _I, _I, _I, _P, _I64, _P, _I64, _P, _P, _U]),
+    "pdk_prefill_attn": (_I, [_P, _I64, _P, _P, _I, _I, _I, _I, _F, _P, _U]),
     "pdk_scatter_koni": (_I, [_P, _I64, _P, _I, _I, _P, _I, _P, _P, _I64, _I, _I, _I, _U]),
     "pdk_host_alloc": (_I, [_SZ, ctypes.POINTER(_P)]),
     "pdk_host_free": (_I, [_P]),

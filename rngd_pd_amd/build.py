@@ -6,8 +6,8 @@ import sys
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _ROOT = os.path.dirname(_HERE)
-SOURCES = ["handoff.hip", "attention.hip", "decode_step.hip", "wgemm.hip", "koni.hip",
-           "staging.hip", "runtime.hip"]
+SOURCES = ["handoff.hip", "attention.hip", "decode_step.hip", "wgemm.hip", "prefill.hip",
+           "koni.hip", "staging.hip", "runtime.hip"]
 OUT = os.path.join(_HERE, "librngdpd.so")
 NET_SOURCES = ["net/tcpkv.cpp"]
 NET_OUT = os.path.join(_HERE, "librngdpd_net.so")
@@ -25,13 +25,14 @@ def hipcc_command(out=OUT):
             + [os.path.join(_HERE, "csrc", s) for s in SOURCES])
 
 
-# Kernels of the handoff and attention paths: a lane's state must fit its
+# Kernels of the handoff, attention and prefill paths: a lane's state must fit its
 # registers. A build in which any of them needs scratch (private) memory is
 # refused: a spill there once cost a serving step 2 ms unnoticed by every
 # correctness test. The decode-step GEMMs for more than 16 streams with wide
 # column groups do spill and are allowed (wgemm_kernel is not listed).
 NO_SCRATCH = ("decode_attn_kernel", "merge_kernel", "pack_kernel", "scatter_kernel",
-              "gather_kernel", "koni_scatter_kernel", "koni_gather_kernel")
+              "gather_kernel", "koni_scatter_kernel", "koni_gather_kernel",
+              "rope_kv_kernel", "prefill_attn_kernel")
 
 
 def resource_report(text):

@@ -9,10 +9,22 @@ done, so saves overlap the layers that follow (the reference emits layer
 groups as it goes).
 
 Prefill is compute-bound (T tokens per weight), so its GEMMs are the
-library's (hipBLASLt through torch); the norms use the decode step's RMSNorm
-kernel; RoPE and causal GQA attention are fp32 torch on contiguous operands.
-Activations are bf16 at tensor boundaries, as in the decode step. It takes
-the decode step's LlamaWeights ([out, in] layout), so a producer and a
+library's (hipBLASLt through torch). Between them, at head_dim 128, one launch
+per line of a layer:
+
+  h = rmsnorm(x + down)                         pdk_rmsnorm, residual add fused
+  qkv = h . Wqkv^T                              library
+  RoPE; K/V rows; attention's operands          pdk_prefill_rope_kv
+  ao = causal GQA attention                     pdk_prefill_attn (fp32 weights)
+  o = ao . Wo^T                                 library
+  h = rmsnorm(x + o)                            pdk_rmsnorm, residual add fused
+  gu = h . Wgu^T                                library
+  act = silu(g) * u                             pdk_swiglu
+  down = act . Wd^T                             library
+
+Other head dims take RoPE and attention as fp32 torch operations on contiguous
+operands. Activations are bf16 at tensor boundaries, as in the decode step. It
+takes the decode step's LlamaWeights ([out, in] layout), so a producer and a
 consumer built from one seed hold the same model.
 """
 import math
@@ -25,6 +37,17 @@ from ..kernels.handoff import stream_handle
 BF16 = torch.bfloat16
 
 
+def _rows(t, shape, device):
+    """The token stride of a layer's K or V rows ([T, Hkv, D] bf16, [Hkv, D]
+    contiguous, 16-byte aligned) as pdk_prefill_rope_kv writes them, or None
+    for any other tensor (filled by a copy instead)."""
+    if t.dtype != BF16 or t.device != device or tuple(t.shape) != shape \
+            or t.data_ptr() % 16 or t.stride(2) != 1 or t.stride(1) != shape[2]:
+        return None
+    ld = t.stride(0) if shape[0] > 1 else shape[1] * shape[2]
+    return ld if ld >= shape[1] * shape[2] and ld % 8 == 0 else None
+
+
 class LlamaPrefill:
     def __init__(self, weights, max_tokens=4096):
         self.w, self.cfg = weights, weights.cfg
@@ -34,10 +57,11 @@ class LlamaPrefill:
         self.inv = cfg.inv_freq().to(self.device)
         self.scale = 1.0 / math.sqrt(cfg.head_dim)
 
-    def _rmsnorm(self, x, weight, out):
+    def _rmsnorm(self, x, weight, out, add=None):
+        """out = rmsnorm(x + add) * weight; with ``add``, x takes the sum."""
         T, H = x.shape
-        _lib.call("pdk_rmsnorm", x.data_ptr(), None, weight.data_ptr(), T, H, self.cfg.eps,
-                  out.data_ptr(), stream_handle())
+        _lib.call("pdk_rmsnorm", x.data_ptr(), None if add is None else add.data_ptr(),
+                  weight.data_ptr(), T, H, self.cfg.eps, out.data_ptr(), stream_handle())
         return out
 
     def _rope(self, t, cos, sin):
@@ -46,6 +70,75 @@ class LlamaPrefill:
         f = t.float()
         a, b = f[..., :half], f[..., half:]
         return torch.cat([a * cos - b * sin, b * cos + a * sin], dim=-1).to(BF16)
+
+    def _kernel_attention(self, T):
+        """The layer's RoPE, KV rows and attention by the HIP kernels: a
+        function (qkv, k_l, v_l, before) -> ao [T, NH HD] bf16; ``before`` is
+        called once k_l and v_l are written."""
+        cfg, dev, st = self.cfg, self.device, stream_handle()
+        NH, NKV, HD = cfg.n_heads, cfg.n_kv_heads, cfg.head_dim
+        table = torch.empty((T, HD // 2, 2), dtype=torch.float32, device=dev)
+        _lib.call("pdk_rope_table", self.inv.data_ptr(), T, HD // 2, table.data_ptr(), st)
+        n = _lib.lib().pdk_prefill_kv_tile_elems(T, NKV)
+        kt, vt = (torch.empty(n, dtype=BF16, device=dev) for _ in range(2))
+        ao = torch.empty((T, NH * HD), dtype=BF16, device=dev)
+
+        def attention(qkv, k_l, v_l, before):
+            rows = []
+            for t in (k_l, v_l):
+                ld = _rows(t, (T, NKV, HD), dev)
+                own = t if ld else torch.empty((T, NKV, HD), dtype=BF16, device=dev)
+                rows.append((own, ld or NKV * HD))
+            (k, k_ld), (v, v_ld) = rows
+            _lib.call("pdk_prefill_rope_kv", qkv.data_ptr(), table.data_ptr(), T, NH, NKV, HD,
+                      k.data_ptr(), k_ld, v.data_ptr(), v_ld, kt.data_ptr(), vt.data_ptr(),
+                      stream_handle())
+            if k is not k_l:
+                k_l.copy_(k)
+            if v is not v_l:
+                v_l.copy_(v)
+            before()
+            _lib.call("pdk_prefill_attn", qkv.data_ptr(), qkv.stride(0), kt.data_ptr(),
+                      vt.data_ptr(), T, NH, NKV, HD, self.scale, ao.data_ptr(), stream_handle())
+            return ao
+
+        return attention
+
+    def _torch_attention(self, T):
+        """The same for head dims the kernels do not take, in fp32 torch."""
+        cfg, dev = self.cfg, self.device
+        NH, NKV, HD = cfg.n_heads, cfg.n_kv_heads, cfg.head_dim
+        G = NH // NKV
+        pos = torch.arange(T, device=dev, dtype=torch.float32)
+        ang = pos[:, None] * self.inv[None, :]                     # fp32 angles, [T, HD/2]
+        cos, sin = torch.cos(ang)[:, None, :], torch.sin(ang)[:, None, :]
+        causal = torch.full((T, T), float("-inf"), device=dev).triu(1)
+
+        def attention(qkv, k_l, v_l, before):
+            q = self._rope(qkv[:, :NH * HD].view(T, NH, HD), cos, sin)
+            k = self._rope(qkv[:, NH * HD:(NH + NKV) * HD].view(T, NKV, HD), cos, sin)
+            v = qkv[:, (NH + NKV) * HD:].view(T, NKV, HD)
+            k_l.copy_(k)
+            v_l.copy_(v)
+            before()
+            # Causal GQA attention in fp32: query head h reads KV head h // G.
+            qf = q.float().view(T, NKV, G, HD).permute(1, 2, 0, 3).reshape(NKV, G * T, HD)
+            kt = k.float().permute(1, 2, 0).contiguous()               # [NKV, HD, T]
+            vf = v.float().permute(1, 0, 2).contiguous()               # [NKV, T, HD]
+            sc = torch.bmm(qf.contiguous(), kt).view(NKV, G, T, T) * self.scale + causal
+            p = torch.softmax(sc, dim=-1).view(NKV, G * T, T)
+            ao = torch.bmm(p, vf).view(NKV, G, T, HD).permute(2, 0, 1, 3).reshape(T, NH * HD)
+            return ao.to(BF16)
+
+        return attention
+
+    def _swiglu(self, gu):
+        T, M = gu.shape[0], self.cfg.inter
+        if M % 8:
+            return (torch.nn.functional.silu(gu[:, :M].float()) * gu[:, M:].float()).to(BF16)
+        act = torch.empty((T, M), dtype=BF16, device=gu.device)
+        _lib.call("pdk_swiglu", gu.data_ptr(), T, M, act.data_ptr(), stream_handle())
+        return act
 
     @torch.no_grad()
     def forward(self, tokens, on_layer=None, kv_out=None):
@@ -57,43 +150,26 @@ class LlamaPrefill:
         T = ids.numel()
         if not 1 <= T <= self.max_tokens:
             raise ValueError(f"prompt of {T} tokens outside [1, {self.max_tokens}]")
-        L, H, NH, NKV, HD = cfg.n_layers, cfg.hidden, cfg.n_heads, cfg.n_kv_heads, cfg.head_dim
-        G, M = NH // NKV, cfg.inter
+        L, H, NKV, HD = cfg.n_layers, cfg.hidden, cfg.n_kv_heads, cfg.head_dim
         if kv_out is None:
             k_all = torch.empty((L, T, NKV, HD), dtype=BF16, device=dev)
             v_all = torch.empty((L, T, NKV, HD), dtype=BF16, device=dev)
         else:
             k_all, v_all = kv_out
-        pos = torch.arange(T, device=dev, dtype=torch.float32)
-        ang = pos[:, None] * self.inv[None, :]                     # fp32 angles, [T, HD/2]
-        cos, sin = torch.cos(ang)[:, None, :], torch.sin(ang)[:, None, :]
-        causal = torch.full((T, T), float("-inf"), device=dev).triu(1)
+        linear = torch.nn.functional.linear
+        attention = (self._kernel_attention if HD == 128 else self._torch_attention)(T)
         x = w.embed.index_select(0, ids)                           # [T, H] bf16
         h = torch.empty_like(x)
+        down = None                                                # not yet added to x
         for li in range(L):
-            self._rmsnorm(x, w.norm1[li], h)
-            qkv = torch.nn.functional.linear(h, w.wqkv[li])         # [T, (NH + 2 NKV) HD]
-            q = self._rope(qkv[:, :NH * HD].view(T, NH, HD), cos, sin)
-            k = self._rope(qkv[:, NH * HD:(NH + NKV) * HD].view(T, NKV, HD), cos, sin)
-            v = qkv[:, (NH + NKV) * HD:].view(T, NKV, HD)
-            k_all[li].copy_(k)
-            v_all[li].copy_(v)
-            if on_layer is not None:
-                on_layer(li, k_all[li], v_all[li])
-            # Causal GQA attention in fp32: query head h reads KV head h // G.
-            qf = q.float().view(T, NKV, G, HD).permute(1, 2, 0, 3).reshape(NKV, G * T, HD)
-            kt = k.float().permute(1, 2, 0).contiguous()               # [NKV, HD, T]
-            vf = v.float().permute(1, 0, 2).contiguous()               # [NKV, T, HD]
-            sc = torch.bmm(qf.contiguous(), kt).view(NKV, G, T, T) * self.scale + causal
-            p = torch.softmax(sc, dim=-1).view(NKV, G * T, T)
-            ao = torch.bmm(p, vf).view(NKV, G, T, HD).permute(2, 0, 1, 3).reshape(T, NH * HD)
-            x = x + torch.nn.functional.linear(ao.to(BF16), w.wo[li])
-            self._rmsnorm(x, w.norm2[li], h)
-            gu = torch.nn.functional.linear(h, w.wgu[li])
-            act = (torch.nn.functional.silu(gu[:, :M].float()) * gu[:, M:].float()).to(BF16)
-            x = x + torch.nn.functional.linear(act, w.wd[li])
+            self._rmsnorm(x, w.norm1[li], h, add=down)
+            k_l, v_l = k_all[li], v_all[li]
+            emit = (lambda: None) if on_layer is None else (lambda: on_layer(li, k_l, v_l))
+            ao = attention(linear(h, w.wqkv[li]), k_l, v_l, emit)
+            self._rmsnorm(x, w.norm2[li], h, add=linear(ao, w.wo[li]))
+            down = linear(self._swiglu(linear(h, w.wgu[li])), w.wd[li])
         last = torch.empty((1, H), dtype=BF16, device=dev)
-        self._rmsnorm(x[T - 1:T].contiguous(), w.norm_f, last)
-        logits = torch.nn.functional.linear(last, w.lm_head)
+        self._rmsnorm(x[T - 1:], w.norm_f, last, add=None if down is None else down[T - 1:])
+        logits = linear(last, w.lm_head)
         first = int(torch.argmax(logits[0]).item())
         return first, k_all, v_all
