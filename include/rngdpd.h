@@ -515,6 +515,16 @@ int pdk_decode_attn_rope_xt(const float* qkv_partials, int splits,
                             uint16_t* out, int plan_batch, uintptr_t stream);
 int pdk_linear_ssq_xt(const uint16_t* x, const uint16_t* wt, int B, int K, int N,
                       const uint16_t* residual, uint16_t* y, float* ssq, uintptr_t stream);
+/* pdk_linear_ssq_xt's result, bit for bit, with a workspace that lets it split
+ * K over workgroups: pdk_linear_ssq_ws_bytes(B, K, N) bytes (0: none needed),
+ * 16-byte aligned, zeroed once before its first use and used by one stream at
+ * a time; the call leaves its counters zero again. A workspace made for a
+ * larger B serves a smaller one. */
+int64_t pdk_linear_ssq_ws_bytes(int B, int K, int N);
+int pdk_linear_ssq_ws_xt(const uint16_t* x, const uint16_t* wt, int B, int K,
+                         int N, const uint16_t* residual, uint16_t* y,
+                         float* ssq, void* workspace, int64_t workspace_bytes,
+                         uintptr_t stream);
 int pdk_linear_swiglu_rms_xt(const uint16_t* x, const uint16_t* wt_gate_up, int B, int K,
                              int M, const float* ssq, int n_ssq, float eps, uint16_t* y,
                              uintptr_t stream);

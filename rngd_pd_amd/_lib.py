@@ -120,6 +120,8 @@ SIGNATURES = {
     "pdk_linear_argmax_rms": (_I, [_P, _P, _I, _I, _I, _P, _I, _F, _P, _P, _P, _U]),
     "pdk_linear_argmax_rms_tiled": (_I, [_P, _P, _I, _I, _I, _P, _I, _F, _P, _P, _P, _U]),
     "pdk_linear_ssq_xt": (_I, [_P, _P, _I, _I, _I, _P, _P, _P, _U]),
+    "pdk_linear_ssq_ws_bytes": (_I64, [_I, _I, _I]),
+    "pdk_linear_ssq_ws_xt": (_I, [_P, _P, _I, _I, _I, _P, _P, _P, _P, _I64, _U]),
     "pdk_linear_swiglu_rms_xt": (_I, [_P, _P, _I, _I, _I, _P, _I, _F, _P, _U]),
     "pdk_linear_splitk_rms_xt": (_I, [_P, _P, _I, _I, _I, _I, _P, _I, _F, _P, _U]),
     "pdk_linear_splitk_final_xt": (_I, [_P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _U]),

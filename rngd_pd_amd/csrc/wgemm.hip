@@ -54,56 +54,13 @@
 
 #include <math.h>
 
-#include "pdk_common.h"
+#include "wgemm_common.h"
 
 namespace {
 
-using pdk::v8;
+using namespace wg;
 
-
-typedef __bf16 bf16x8_t __attribute__((__vector_size__(16)));
-typedef float f32x4 __attribute__((__vector_size__(16)));
-
-__device__ __forceinline__ f32x4 mfma(const v8& a, const v8& b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                 __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
-
-constexpr int kStepK = 128;        // k per wave step: 4 MFMA of 32
 constexpr int kWaves = 8;
-constexpr int kBlock = 16 * kStepK;  // tiled W: one tile's k step, 4 KiB
-
-// kResidualSsq: kResidual that also writes, per 16-column tile and row, the
-// sum of squares of the bf16 outputs (ssq[row][tile]): the raw material of the
-// next RMSNorm. kSwiGLURms: kSwiGLU on weights with that norm's gain folded
-// into their columns, whose input x is the un-normalised residual: each row's
-// two sums are scaled by r = rsqrt(sum(ssq[row][.]) / K + eps) before SwiGLU,
-// so rmsnorm(x) . W^T = r * (x . (W diag g)^T) takes no launch of its own.
-//
-// kPartialFinal: kPartial whose last-arriving split of each column group adds
-// the splits' partials in split order to the residual (y = bf16(r + sum), r
-// may alias y: the update pdk_rmsnorm_partials makes) and writes that
-// group's sums of squares as kResidualSsq does, so the next RMSNorm needs no
-// launch. kArgmaxRms: kArgmax on weights with the final norm's gain folded in,
-// each row's logits scaled by its r (from ssq) before rounding. kPartialRms:
-// kPartial on weights with a norm's gain folded in, each row's partial scaled
-// by its r (the q|k|v projection: its consumer adds the scaled halves).
-enum Epilogue { kPlain = 0, kResidual = 1, kSwiGLU = 2, kArgmax = 3, kPartial = 4,
-                kResidualSsq = 5, kSwiGLURms = 6, kPartialFinal = 7, kArgmaxRms = 8,
-                kPartialRms = 9 };
-
-// Greedy-token key of one bf16 logit: the value in an order-preserving code
-// above the complement of the column, so the unsigned maximum is the largest
-// value at its lowest column (torch.argmax: NaN above every number, the first
-// of equal values; -0 counts as +0). 0 is below every key.
-__device__ __forceinline__ uint64_t argmax_key(uint32_t h, int n) {
-  h &= 0xffffu;
-  if (h == 0x8000u) h = 0;                                   // -0 -> +0
-  uint32_t ord;
-  if ((h & 0x7fffu) > 0x7f80u) ord = 0xffffu;               // NaN
-  else ord = (h & 0x8000u) ? (~h & 0xffffu) : (h | 0x8000u);
-  return ((uint64_t)ord << 32) | (uint64_t)(0xffffffffu - (uint32_t)n);
-}
 
 // Loads in flight per wave: kDepth steps of W (and X), no more than about 160
 // VGPRs of load buffers, and at most 4. With step-major tiled weights fewer
@@ -337,10 +294,10 @@ __global__ __launch_bounds__(kWaves * 64) void wgemm_kernel(const uint16_t* __re
       float v[kPairs];
 #pragma unroll
       for (int p = 0; p < kPairs; ++p) {
-        float sum = 0.f;
+        float cls[kWaves];                       // wave q holds step class q
 #pragma unroll
-        for (int q = 0; q < kWaves; ++q) sum += red[q][p * kCols + c][e & 255];
-        v[p] = sum;
+        for (int q = 0; q < kWaves; ++q) cls[q] = red[q][p * kCols + c][e & 255];
+        v[p] = sum_classes<kEpi>(cls);
       }
       // Logits (the argmax epilogues) stay row-major; y and the residual are
       // activations, tiled with kAct.
@@ -491,11 +448,15 @@ int launch_cols(const uint16_t* x, const uint16_t* w, int B, int K, int N, const
   const dim3 grid((N + 16 * kCols - 1) / (16 * kCols), splits), block(kWaves * 64);
 #define PDK_WGEMM(T) \
   hipLaunchKernelGGL((wgemm_kernel<T, kCols, kEpi, kTiled, kAct>), grid, block, 0, st, x, w, B, K, N, splits, ssq, r, y, keys, part, eps, counters)
-  switch ((B + 15) / 16) {
-    case 1: PDK_WGEMM(1); break;
-    case 2: PDK_WGEMM(2); break;
-    case 3: PDK_WGEMM(3); break;
-    default: PDK_WGEMM(4); break;
+  if constexpr (kCols == 8) {                          // at most 16 rows (see launch)
+    PDK_WGEMM(1);
+  } else {
+    switch ((B + 15) / 16) {
+      case 1: PDK_WGEMM(1); break;
+      case 2: PDK_WGEMM(2); break;
+      case 3: PDK_WGEMM(3); break;
+      default: PDK_WGEMM(4); break;
+    }
   }
 #undef PDK_WGEMM
   return pdk::check_launch("wgemm_kernel");
@@ -511,16 +472,40 @@ int launch(const uint16_t* x, const uint16_t* w, int B, int K, int N, const uint
            uint16_t* y, uint64_t* keys, hipStream_t st, float* ssq = nullptr, int n_ssq = 0,
            float eps = 0.f) {
   const int64_t wide = (N + 63) / 64;                // workgroups with 4 tiles
+  if constexpr (kAct && kEpi == kSwiGLURms) {
+    if (wide_swiglu(B, K, N)) return launch_wide_swiglu(x, w, B, K, N, ssq, eps, y, st);
+    // Beyond 32 streams two tiles (four weight tiles per step) still fit the
+    // registers: 66.9 us with one tile, 52.8 with two at B = 50, M = 14336.
+    if (B > 32 && wide >= 192)
+      return launch_cols<2, kEpi, kTiled, kAct>(x, w, B, K, N, r, y, keys, st, nullptr, 1, ssq,
+                                                n_ssq, eps);
+  }
+  // The lm_head on tiled operands, K = 4096 (us, columns per workgroup 16 / 32
+  // / 64 / 128): N = 8016 B=1 15.6 / 16.5 / 18.9 / 27.6, B=16 21.7 / 18.5 / 20.7
+  // / 29.0, B=50 36.7 / 26.7 / 29.5 / -; N = 16032 B=1 32.9 / 29.0 / 26.2 / 32.9,
+  // B=16 36.8 / 31.6 / 28.8 / 34.6, B=50 65.2 / 44.7 / 36.6 / -; N = 32064 B=1
+  // 54.8 / 53.7 / 49.6 / 49.1, B=16 63.2 / 56.6 / 52.9 / 48.8; N = 128256 B=16
+  // 215 / 194 / 178 / 174, B=20 308 / 222 / 195 / 213. So the widest that leaves
+  // about 200 workgroups, except that one tile is best for a few rows, and 8
+  // tiles only up to 16 rows (more rows leave no registers).
+  if constexpr (kAct && kEpi == kArgmaxRms) {
+    if (wide_argmax(B, K, N)) return launch_wide_argmax(x, w, B, K, N, ssq, eps, y, keys, st);
+    if (B <= 16 && wide >= 448)
+      return launch_cols<8, kEpi, kTiled, kAct>(x, w, B, K, N, r, y, keys, st, nullptr, 1, ssq,
+                                                n_ssq, eps);
+    if (wide >= 192)
+      return launch_cols<4, kEpi, kTiled, kAct>(x, w, B, K, N, r, y, keys, st, nullptr, 1, ssq,
+                                                n_ssq, eps);
+    if (B >= 8 && wide >= 96)
+      return launch_cols<2, kEpi, kTiled, kAct>(x, w, B, K, N, r, y, keys, st, nullptr, 1, ssq,
+                                                n_ssq, eps);
+    return launch_cols<1, kEpi, kTiled, kAct>(x, w, B, K, N, r, y, keys, st, nullptr, 1, ssq,
+                                              n_ssq, eps);
+  }
   // Wide SwiGLU tiles hold 8 weight tiles per step in registers: beyond 32
-  // streams they would spill, and one tile is used instead. The lm_head with
+  // streams they would spill, and fewer tiles are used instead. The lm_head with
   // tiled weights runs 4 tiles wide at every B (B = 4: 181 -> 178 us).
   constexpr bool kGLU = kEpi == kSwiGLU || kEpi == kSwiGLURms;
-  // The lm_head on tiled activations runs 8 tiles wide up to B = 32: each
-  // workgroup reads the activation rows once for 128 columns instead of 64,
-  // and the decode step at B = 16 went 3.022 -> 3.007 ms (B = 4 unchanged).
-  if (kAct && kEpi == kArgmaxRms && B <= 32 && wide >= 1024)
-    return launch_cols<8, kEpi, kTiled, kAct>(x, w, B, K, N, r, y, keys, st, nullptr, 1, ssq,
-                                              n_ssq, eps);
   const bool four = kGLU ? (wide >= 192 && B <= 32) : ((B > 8 || kTiled) && wide >= 1024);
   if (four) return launch_cols<4, kEpi, kTiled, kAct>(x, w, B, K, N, r, y, keys, st, nullptr, 1,
                                                       ssq, n_ssq, eps);
@@ -839,6 +824,29 @@ extern "C" int pdk_linear_ssq_xt(const uint16_t* x, const uint16_t* wt, int B, i
                                  const uint16_t* residual, uint16_t* y, float* ssq,
                                  uintptr_t stream) {
   return linear_ssq<true, true>(x, wt, B, K, N, residual, y, ssq, stream);
+}
+
+extern "C" int64_t pdk_linear_ssq_ws_bytes(int B, int K, int N) {
+  if (B < 1 || B > 64 || N < 1 || !wide_ssq(B, K, N)) return 0;
+  return (int64_t)kWideSplits * B * N * 4 + (int64_t)((N + 63) / 64) * 4;
+}
+
+extern "C" int pdk_linear_ssq_ws_xt(const uint16_t* x, const uint16_t* wt, int B, int K, int N,
+                                    const uint16_t* residual, uint16_t* y, float* ssq,
+                                    void* workspace, int64_t workspace_bytes, uintptr_t stream) {
+  pdk::clear_error();
+  if (int rc = check_shape(x, wt, y, B, K, N)) return rc;
+  const int64_t need = pdk_linear_ssq_ws_bytes(B, K, N);
+  if (need == 0) return linear_ssq<true, true>(x, wt, B, K, N, residual, y, ssq, stream);
+  PDK_REQUIRE(residual && ssq, "null pointer argument");
+  PDK_REQUIRE(N % kStepK == 0, "tiled activations need N %% %d == 0 (got %d)", kStepK, N);
+  PDK_REQUIRE(workspace && workspace_bytes >= need && pdk::aligned16(workspace),
+              "workspace of %lld bytes needed (got %lld)", (long long)need,
+              (long long)workspace_bytes);
+  // The counters come first: their place then does not depend on B.
+  int* counters = static_cast<int*>(workspace);
+  float* part = reinterpret_cast<float*>(counters + (N + 63) / 64);
+  return launch_wide_ssq(x, wt, B, K, N, residual, y, ssq, part, counters, pdk::as_stream(stream));
 }
 
 extern "C" int pdk_linear_swiglu_rms_xt(const uint16_t* x, const uint16_t* wt_gate_up, int B,

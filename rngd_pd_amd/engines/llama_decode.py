@@ -173,6 +173,11 @@ class LlamaDecoder:
         # 8B step took as long at B = 16 (2.923-2.925 against 2.920-2.927 ms)
         # and 34 us longer at B = 4 (2.767-2.770 against 2.733-2.738), in one
         # process with step-major tiled weights.
+        # Beyond 16 streams on tiled operands the down projection does split K,
+        # over four workgroups per 64 columns (pdk_linear_ssq_ws_xt, the same
+        # bits): 35.7 -> 27.0 us at B = 50. Its workspace starts zeroed.
+        ws = _lib.lib().pdk_linear_ssq_ws_bytes(B, cfg.inter, H) if self.act_tiled else 0
+        self.down_ws = torch.zeros(-(-ws // 4), dtype=torch.int32, device=dev) if ws else None
         # The q|k|v projection (N = 6144 at 8B) splits K in two when every wave
         # of the GEMM still gets two 128-long steps of each half: 2 x 96 wide
         # workgroups instead of 384 narrow ones, which re-read x per 16
@@ -291,6 +296,8 @@ class LlamaDecoder:
         lin_ssq, lin_swr, lin_amr = (g["pdk_linear_ssq"], g["pdk_linear_swiglu_rms"],
                                      g["pdk_linear_argmax_rms"])
         ssqp, ssqa, n_ssq = self.ssq.data_ptr(), self.ssq_a.data_ptr(), H // 16
+        down_ws = None if self.down_ws is None else (self.down_ws.data_ptr(),
+                                                     self.down_ws.numel() * 4)
         emb, attn = g["pdk_embed_ssq"], g["pdk_decode_attn_rope"]
         with torch.cuda.stream(stream) if stream is not None else contextlib.nullcontext():
             call(emb, w.embed.data_ptr(), cfg.vocab, tokens.data_ptr(),
@@ -302,7 +309,10 @@ class LlamaDecoder:
                      B, NH, NKV, HD, self.scale, ws_ptr, ws_bytes, aop, self.plan_batch, st)
                 call(lin_ssq, aop, wo, B, NH * HD, H, xp, xp, ssqp, st)
                 call(lin_swr, xp, wgu, B, H, M, ssqp, n_ssq, eps, actp, st)
-                call(lin_ssq, actp, wd, B, M, H, xp, xp, ssqa, st)
+                if down_ws is None:
+                    call(lin_ssq, actp, wd, B, M, H, xp, xp, ssqa, st)
+                else:
+                    call("pdk_linear_ssq_ws_xt", actp, wd, B, M, H, xp, xp, ssqa, *down_ws, st)
             call(lin_amr, xp, self._lm_head.data_ptr(), B, H, cfg.vocab, ssqa, n_ssq, eps,
                  self.logits.data_ptr(), self.keys.data_ptr(), self.tokens.data_ptr(), st)
         return self.tokens[:B]
