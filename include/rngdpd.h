@@ -200,6 +200,20 @@ int pdk_decode_attn(const uint16_t* q, const uint16_t* cache_k,
                     void* workspace, size_t workspace_bytes, uint16_t* out,
                     uintptr_t stream);
 
+/* pdk_cache_append followed by pdk_decode_attn, in one launch and with the
+ * same results, bit for bit: the new token's k_new and v_new [B][n_kv_heads]
+ * [head_dim] (16-byte aligned) go to slot ctx_lens[b] - 1 of the cache and
+ * take part in the attention. No two streams may share that slot's block. */
+int pdk_decode_attn_append(const uint16_t* q, const uint16_t* k_new,
+                           const uint16_t* v_new, uint16_t* cache_k,
+                           uint16_t* cache_v, int num_blocks,
+                           const int32_t* block_tables, int max_blocks,
+                           const int32_t* ctx_lens, int max_ctx, int B,
+                           int n_q_heads, int n_kv_heads, int head_dim,
+                           float scale, void* workspace,
+                           size_t workspace_bytes, uint16_t* out,
+                           uintptr_t stream);
+
 /* pdk_decode_attn without the workspace argument, for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc). No counterpart in the reference. The split

@@ -379,6 +379,13 @@ __device__ __forceinline__ void attend_span(const AttnArgs& a, Span& r, const v8
 // them for the new token in place of the cache's contents. Every value is the
 // one pdk_rope_cache_append_partials computes, so the result is bit-identical
 // to that kernel followed by the kRope = 0 path.
+// kRope = kAppend: src is q as with 0, and the new token's k and v come as bf16
+// [B][Hkv][D] rows (k_new, v_new): into LDS, to their cache slot and into the
+// span that holds the position as with the fused RoPE. The result is that of
+// pdk_cache_append followed by the kRope = 0 path, bit for bit, without the
+// append's launch: per layer (32 query, 8 KV heads, HIP graph) B=16 ctx 512 11.0
+// -> 9.1 us, B=8 ctx 512 10.0 -> 8.4, B=16 ctx 4096 52.6 -> 50.4, B=1 ctx 8192
+// 17.3 -> 15.0, B=64 ctx 1024 (8 query heads) 51.6 -> 51.9.
 // kRope = -1 is the read probe (pdk_attn_read_probe): the same launch, block
 // ids and K/V loads, none of the arithmetic, one store per thread.
 // kAct: out in the decode step's tiled activation layout (pdk::act_at, row b,
@@ -390,17 +397,21 @@ __device__ __forceinline__ void attend_span(const AttnArgs& a, Span& r, const v8
 // load between two alternative instructions, and the compiler's wait counts
 // then ignore the loads on both sides of that choice: every K/V wait of the
 // wavefront became a wait for nearly all of its loads.
+constexpr int kAppend = 8;
+
 template <int kRope, int kNV, bool kAct = false, bool kKnt = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_attn_kernel(
     const void* src, const uint16_t* ck, const uint16_t* cv, const int32_t* tables,
     const int32_t* ctx_lens, uint32_t hgw, uint32_t mb_b, int num_blocks, uint32_t st_ns,
     float scale_log2, uint16_t* out, float* ws_ml, float* ws_o, const float* inv_freq,
-    uint16_t* ck_w, uint16_t* cv_w, const float* ssq, int n_ssq, float eps) {
+    uint16_t* ck_w, uint16_t* cv_w, const float* ssq, int n_ssq, float eps,
+    const uint16_t* k_new, const uint16_t* v_new) {
+  constexpr bool kRot = kRope > 0 && kRope != kAppend;   // the fused RoPE
   const uint16_t* q = static_cast<const uint16_t*>(src);
   const float* part = static_cast<const float*>(src);
   __shared__ __align__(16) float sm_m[kMaxG][kMaxWaves];
   __shared__ __align__(16) float sm_l[kMaxG][kMaxWaves];
-  __shared__ __align__(16) uint16_t q_rot[kRope ? kMaxG : 1][kD];   // rotated q of the group
+  __shared__ __align__(16) uint16_t q_rot[kRot ? kMaxG : 1][kD];   // rotated q of the group
   __shared__ __align__(16) uint16_t kv_new[2][kD];                  // rotated k, v of the new token
   extern __shared__ float sm_o[];                // [min(G, kMergeRows)][kORow]
 
@@ -419,9 +430,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // plain path B=16 8.71 -> 8.37 us, B=8 6.98 -> 6.75, B=4 6.06 -> 5.88; on
   // the fused RoPE path no faster, and 0.15-0.3 us slower between streaming
   // kernels, so it keeps ordinary loads.
-  constexpr bool kVStream = kRope <= 0;
+  constexpr bool kVStream = !kRot;
   const int qsplit = hgw >> 24;
-  static_assert(!kKnt || (kRope <= 0 && kNV == 4), "non-temporal K only on the plain V-split path");
+  static_assert(!kKnt || (!kRot && kNV == 4), "non-temporal K only on the plain V-split path");
   constexpr bool knt = kKnt;
   const int gs = qsplit + kVS;                   // log2 of the workgroups sharing a unit
   const int units = nsplit * a.Hkv * (int)(mb_b >> 16);
@@ -448,7 +459,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int32_t* table = a.tables + (int64_t)b * a.max_blocks;
 
   v8 qv[4];
-  if constexpr (kRope == 0) {
+  if constexpr (kRope == 0 || kRope == kAppend) {
     const uint16_t* qp = a.q + ((int64_t)b * a.Hq + qh0 + min(j, G - 1)) * kD + g * 8;
 #pragma unroll
     for (int s = 0; s < 4; ++s) qv[s] = pdk::ld16(qp + 32 * s);
@@ -479,7 +490,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // query heads (dims lane and lane + 64), r == G the new k, r == G+1, G+2 the
   // new v (dims 64 (r - G - 1) + lane); row r belongs to wavefront r % W.
   constexpr int kPre = 4;                        // rows per wavefront loaded early
-  constexpr int kParts = kRope > 0 ? kRope : 1;
+  constexpr int kParts = kRot ? kRope : 1;
   const int n_rows = G + 3;
   const int64_t n_qkv = (int64_t)(a.Hq + 2 * a.Hkv) * kD;
   const int64_t part_stride = (int64_t)(mb_b >> 16) * n_qkv;   // one split of the partials
@@ -492,7 +503,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   float raw[kPre][2][kParts];
   float ifreq = 0.f;
   pdk::RowRms rr{};
-  if constexpr (kRope > 0) {
+  if constexpr (kRot) {
 #pragma unroll
     for (int k = 0; k < kPre; ++k) {
       const int r = wv + k * W;
@@ -526,9 +537,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // block ids; the row scale's loads and the frequencies go out after the
   // partial sums' and before any K/V load (a wavefront's loads complete in
   // order), and the scale is finished after the K/V loads are issued.
-  if constexpr (kRope > 0) {
+  if constexpr (kRot) {
     if (ssq) rr = pdk::row_rms_load(ssq, b, n_ssq, lane);
     ifreq = inv_freq[lane];
+  }
+  // The new token's k (lanes 0-15, 8 dims each) and v (lanes 16-31), ahead of
+  // every K/V load; the other lanes repeat them.
+  v8 fresh = pdk::zero8();
+  if constexpr (kRope == kAppend) {
+    const int64_t row = ((int64_t)b * a.Hkv + h) * kD + (lane & 15) * 8;
+    fresh = pdk::ld16((lane & 16 ? v_new : k_new) + row);
   }
   const int ctx = min(ctx_raw, a.max_blocks * 16);
   const int s_end = (split == a.nsplit - 1) ? ctx : min(ctx, s_begin + a.split_tokens);
@@ -558,7 +576,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // barrier after the rotation keeps every wavefront on one path up to it);
   // on the other paths such a wavefront skips the loads and the spans at once.
   if constexpr (kRope > 0) first_loads();
-  if constexpr (kRope > 0) {
+  if constexpr (kRope == kAppend) {
+    if (wv == 0 && lane < 32)
+      *reinterpret_cast<v8*>(&kv_new[lane >> 4][(lane & 15) * 8]) = fresh;
+    __syncthreads();
+  }
+  if constexpr (kRot) {
     // Second phase, while the first pair's K/V loads are in flight: add the
     // partials in split order, round to bf16 (the projection's output), rotate
     // q and k with the angle pos * inv_freq[lane], and put the group's q and
@@ -608,6 +631,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int s = 0; s < 4; ++s)
       qv[s] = *reinterpret_cast<const v8*>(&q_rot[min(j, G - 1)][32 * s + 8 * g]);
+  }
+  if constexpr (kRope > 0) {
     // The new token's k and v into its cache slot, by one wavefront of the
     // unit's first workgroup (part 0), in the split that holds the position: issued now, behind every K/V load of the wavefront, the
     // stores complete while the loads' data arrives (the spans that hold the
@@ -937,6 +962,8 @@ struct RopeIn {
   int n_ssq = 0;
   float eps = 0.f;
   bool probe = false;            // pdk_attn_read_probe: loads only
+  const uint16_t* k_new = nullptr;   // pdk_decode_attn_append: the new token's rows
+  const uint16_t* v_new = nullptr;
   bool act = false;              // out in the tiled activation layout (pdk::act_at)
 };
 
@@ -944,7 +971,7 @@ struct RopeIn {
 // probe non-temporal K when the two V halves are K's only readers.
 template <int kRope, bool kAct>
 auto attn_kernel_for(const Plan& p) {
-  if constexpr (kRope <= 0) {
+  if constexpr (kRope <= 0 || kRope == kAppend) {
     if (p.vsplit && p.qsplit == 0) return decode_attn_kernel<kRope, 4, kAct, true>;
   }
   return p.vsplit ? decode_attn_kernel<kRope, 4, kAct, false> : decode_attn_kernel<kRope, 8, kAct, false>;
@@ -1024,9 +1051,10 @@ int launch_attn(const uint16_t* q, const uint16_t* cache_k, const uint16_t* cach
     const auto kern = attn_kernel_for<R, A>(p);                                                \
     hipLaunchKernelGGL(kern, grid, block, lds, st, src, a.ck, a.cv, a.tables, a.ctx, hgw, mb_b, \
                        a.num_blocks, st_ns, a.scale_log2, a.out, a.ws_ml, a.ws_o,              \
-                       rope.inv_freq, rope.ck_w, rope.cv_w, rope.ssq, rope.n_ssq, rope.eps);   \
+                       rope.inv_freq, rope.ck_w, rope.cv_w, rope.ssq, rope.n_ssq, rope.eps,    \
+                       rope.k_new, rope.v_new);                                                \
   } while (0)
-  const int mode = rope.probe ? -1 : rope.part ? rope.splits : 0;
+  const int mode = rope.probe ? -1 : rope.part ? rope.splits : rope.k_new ? kAppend : 0;
   if (rope.act) {
     switch (mode) {
       case 1: PDK_ATTN_LAUNCH(1, true); break;
@@ -1043,6 +1071,7 @@ int launch_attn(const uint16_t* q, const uint16_t* cache_k, const uint16_t* cach
       case 1: PDK_ATTN_LAUNCH(1, false); break;
       case 2: PDK_ATTN_LAUNCH(2, false); break;
       case 4: PDK_ATTN_LAUNCH(4, false); break;
+      case kAppend: PDK_ATTN_LAUNCH(kAppend, false); break;
       default:
         pdk::set_error("splits must be 1, 2 or 4 (got %d)", rope.splits);
         return PDK_EINVAL;
@@ -1072,6 +1101,35 @@ extern "C" int pdk_decode_attn(const uint16_t* q, const uint16_t* cache_k, const
   return launch_attn(q, cache_k, cache_v, num_blocks, block_tables, max_blocks, ctx_lens, max_ctx,
                      B, n_q_heads, n_kv_heads, head_dim, scale, workspace, workspace_bytes, out,
                      stream, RopeIn{nullptr, 0, nullptr, nullptr, nullptr}, B);
+}
+
+extern "C" int pdk_decode_attn_append(const uint16_t* q, const uint16_t* k_new,
+                                      const uint16_t* v_new, uint16_t* cache_k, uint16_t* cache_v,
+                                      int num_blocks, const int32_t* block_tables, int max_blocks,
+                                      const int32_t* ctx_lens, int max_ctx, int B, int n_q_heads,
+                                      int n_kv_heads, int head_dim, float scale, void* workspace,
+                                      size_t workspace_bytes, uint16_t* out, uintptr_t stream) {
+  pdk::clear_error();
+  PDK_REQUIRE(q && k_new && v_new, "null pointer argument");
+  PDK_REQUIRE(pdk::aligned16(k_new) && pdk::aligned16(v_new), "k_new/v_new must be 16-byte aligned");
+  // With several rounds of workgroups that read next to nothing each, every
+  // round's wait for the new rows costs more than the append's launch: B=64, 8
+  // KV heads, ctx 64 11.6 us per layer in two launches, 12.6 in one; ctx 256 20.6
+  // and 18.8.
+  if ((int64_t)B * n_kv_heads > kTargetWorkgroups && max_ctx <= 128) {
+    if (int rc = pdk_cache_append(k_new, v_new, cache_k, cache_v, num_blocks, block_tables,
+                                  max_blocks, ctx_lens, B, n_kv_heads, head_dim, stream))
+      return rc;
+    return pdk_decode_attn(q, cache_k, cache_v, num_blocks, block_tables, max_blocks, ctx_lens,
+                           max_ctx, B, n_q_heads, n_kv_heads, head_dim, scale, workspace,
+                           workspace_bytes, out, stream);
+  }
+  RopeIn in{nullptr, 0, nullptr, cache_k, cache_v};
+  in.k_new = k_new;
+  in.v_new = v_new;
+  return launch_attn(q, cache_k, cache_v, num_blocks, block_tables, max_blocks, ctx_lens, max_ctx,
+                     B, n_q_heads, n_kv_heads, head_dim, scale, workspace, workspace_bytes, out,
+                     stream, in, B);
 }
 
 extern "C" int pdk_decode_attn_noalloc(const uint16_t* q, const uint16_t* cache_k,

@@ -69,12 +69,12 @@ class BatchDecodeAttention:
         """One layer: write the new token's k/v at slot pos, attend over 0..pos.
         q [B, Hq, D], k_new/v_new [B, Hkv, D] bf16 on the device."""
         ck, cv = self.cache.k[layer], self.cache.v[layer]
-        _attn.cache_append(k_new, v_new, ck, cv, tables, ctx, stream=stream)
         need = _attn.workspace_bytes(q.shape[0], self.Hq, max_ctx, self.cache.head_dim)
         if need and (self._ws is None or self._ws.numel() * 4 < need):
             self._ws = torch.zeros(need // 4 + 64, dtype=torch.float32, device=self.cache.device)
-        return _attn.decode_attention(q, ck, cv, tables, ctx, max_ctx, scale=self.scale, out=out,
-                                      workspace=self._ws if need else None, stream=stream)
+        return _attn.decode_attention_append(q, k_new, v_new, ck, cv, tables, ctx, max_ctx,
+                                             scale=self.scale, out=out,
+                                             workspace=self._ws if need else None, stream=stream)
 
     def advance(self, req_ids):
         """After all layers of a step: every stream moves to its next position."""

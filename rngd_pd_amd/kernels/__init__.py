@@ -2,7 +2,8 @@
 from .handoff import (pack_kv, pack_kv_batch, scatter_paged, scatter_paged_batch, gather_paged,
                       frame_shape, frame_views, stream_handle, validate_table, copy_kernel,
                       stream_probe, check_skipped)
-from .attention import (decode_attention, decode_attention_rope, cache_append, greedy_argmax,
+from .attention import (decode_attention, decode_attention_append, decode_attention_rope,
+                        cache_append, greedy_argmax,
                         workspace_bytes, get_workspace, attn_read_probe)
 from .decode_step import (rmsnorm, rope_cache_append, rope_cache_append_partials, swiglu, linear,
                           linear_swiglu, linear_argmax, linear_splitk, rmsnorm_partials,
@@ -14,7 +15,8 @@ __all__ = ["pack_kv", "pack_kv_batch", "scatter_paged", "scatter_paged_batch", "
            "frame_shape", "frame_views", "stream_handle", "validate_table", "copy_kernel",
            "check_skipped",
            "stream_probe",
-           "decode_attention", "decode_attention_rope", "cache_append", "greedy_argmax", "workspace_bytes", "get_workspace",
+           "decode_attention", "decode_attention_append", "decode_attention_rope",
+           "cache_append", "greedy_argmax", "workspace_bytes", "get_workspace",
            "attn_read_probe",
            "rmsnorm", "rope_cache_append", "rope_cache_append_partials", "swiglu", "linear", "linear_swiglu", "linear_argmax",
            "linear_splitk", "rmsnorm_partials", "linear_ssq", "linear_swiglu_rms", "fold_norm",

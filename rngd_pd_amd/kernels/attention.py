@@ -47,13 +47,9 @@ def _check_layer_cache(cache_k, cache_v):
     return nb, H, D
 
 
-def decode_attention(q, cache_k, cache_v, block_tables, ctx_lens, max_ctx, scale=1.0,
-                     out=None, workspace=None, stream=None):
-    """GQA decode attention for one layer.
-
-    q [B, Hq, D] bf16 (query head h reads KV head h // (Hq/Hkv)); cache_k
-    [nb, Hkv, 16, D] (tiled K blocks), cache_v [nb, Hkv, D, 16]; block_tables int32 [B, max_blocks]
-    and ctx_lens int32 [B] on the device; ``max_ctx`` >= every ctx_lens[b]."""
+def _attention_call(q, cache_k, cache_v, block_tables, ctx_lens, max_ctx, out, workspace):
+    """Checked operands of one attention call: (geometry, workspace pointer and
+    bytes, out)."""
     _need(q, "q")
     nb, H, D = _check_layer_cache(cache_k, cache_v)
     if q.dim() != 3 or q.shape[2] != D or not q.is_contiguous():
@@ -78,9 +74,46 @@ def decode_attention(q, cache_k, cache_v, block_tables, ctx_lens, max_ctx, scale
             ws = get_workspace(need, q.device)
     ws_ptr = ws.data_ptr() if ws is not None else None
     ws_bytes = ws.numel() * ws.element_size() if ws is not None else 0
+    return (nb, B, Hq, H, D), ws_ptr, ws_bytes, out
+
+
+def decode_attention(q, cache_k, cache_v, block_tables, ctx_lens, max_ctx, scale=1.0,
+                     out=None, workspace=None, stream=None):
+    """GQA decode attention for one layer.
+
+    q [B, Hq, D] bf16 (query head h reads KV head h // (Hq/Hkv)); cache_k
+    [nb, Hkv, 16, D] (tiled K blocks), cache_v [nb, Hkv, D, 16]; block_tables int32 [B, max_blocks]
+    and ctx_lens int32 [B] on the device; ``max_ctx`` >= every ctx_lens[b]."""
+    (nb, B, Hq, H, D), ws_ptr, ws_bytes, out = _attention_call(
+        q, cache_k, cache_v, block_tables, ctx_lens, max_ctx, out, workspace)
     _lib.call("pdk_decode_attn", q.data_ptr(), cache_k.data_ptr(), cache_v.data_ptr(), nb,
               block_tables.data_ptr(), block_tables.shape[1], ctx_lens.data_ptr(), int(max_ctx),
               B, Hq, H, D, float(scale), ws_ptr, ws_bytes, out.data_ptr(), stream_handle(stream))
+    return out
+
+
+def decode_attention_append(q, k_new, v_new, cache_k, cache_v, block_tables, ctx_lens, max_ctx,
+                            scale=1.0, out=None, workspace=None, stream=None):
+    """cache_append(k_new, v_new) then decode_attention, in one launch where the
+    kernel takes it (head_dim 128, 16-byte aligned rows), with the same results
+    bit for bit. k_new, v_new bf16 [B, Hkv, D]."""
+    _need(k_new, "k_new")
+    _need(v_new, "v_new")
+    nb, H, D = _check_layer_cache(cache_k, cache_v)
+    B = k_new.shape[0]
+    if tuple(k_new.shape) != (B, H, D) or tuple(v_new.shape) != (B, H, D):
+        raise ValueError("k_new/v_new must be [B, Hkv, D]")
+    k_new, v_new = k_new.contiguous(), v_new.contiguous()
+    if D != 128 or B != q.shape[0] or k_new.data_ptr() % 16 or v_new.data_ptr() % 16:
+        cache_append(k_new, v_new, cache_k, cache_v, block_tables, ctx_lens, stream=stream)
+        return decode_attention(q, cache_k, cache_v, block_tables, ctx_lens, max_ctx, scale=scale,
+                                out=out, workspace=workspace, stream=stream)
+    (nb, B, Hq, H, D), ws_ptr, ws_bytes, out = _attention_call(
+        q, cache_k, cache_v, block_tables, ctx_lens, max_ctx, out, workspace)
+    _lib.call("pdk_decode_attn_append", q.data_ptr(), k_new.data_ptr(), v_new.data_ptr(),
+              cache_k.data_ptr(), cache_v.data_ptr(), nb, block_tables.data_ptr(),
+              block_tables.shape[1], ctx_lens.data_ptr(), int(max_ctx), B, Hq, H, D, float(scale),
+              ws_ptr, ws_bytes, out.data_ptr(), stream_handle(stream))
     return out
 
 
