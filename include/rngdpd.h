@@ -691,6 +691,38 @@ int pdk_prefill_rope_kv(uint16_t* qkv, const float* table, int T, int n_q_heads,
                         int64_t v_tok_stride, uint16_t* kt, uint16_t* vt,
                         uintptr_t stream);
 
+/* The projections of prompts of up to 256 tokens (512 where N is small enough
+ * that the library's tiles would leave the chip idle): W [N][K] bf16 as the
+ * model holds it, K split over workgroups. pdk_prefill_gemm_splits: how many
+ * splits T, K, N give, 0 where pdk_prefill_gemm does not take them (K % 64, N %
+ * 4, K >= 256, or a shape the library is faster at). pdk_prefill_gemm writes
+ * that many fp32 partial sums, partials [splits][T][N], for
+ * pdk_prefill_rope_kv_partials or pdk_prefill_rmsnorm_partials.
+ * pdk_prefill_gemm_swiglu (where pdk_prefill_gemm_swiglu_takes is 1): y [T][M]
+ * = silu(x . Wg^T) * (x . Wu^T) from w_gate_up = [Wg; Wu] [2M][K], rounded once. */
+int pdk_prefill_gemm_splits(int T, int K, int N);
+int pdk_prefill_gemm(const uint16_t* x, const uint16_t* w, int T, int K, int N,
+                     float* partials, uintptr_t stream);
+int pdk_prefill_gemm_swiglu_takes(int T, int K, int M);
+int pdk_prefill_gemm_swiglu(const uint16_t* x, const uint16_t* w_gate_up, int T,
+                            int K, int M, uint16_t* y, uintptr_t stream);
+
+/* pdk_prefill_rope_kv on the projection's partial sums (added in order, rounded
+ * to bf16 once); the rotated q goes to q_out [T][Hq][128]. */
+int pdk_prefill_rope_kv_partials(const float* partials, int splits,
+                                 const float* table, int T, int n_q_heads,
+                                 int n_kv_heads, int head_dim, uint16_t* q_out,
+                                 uint16_t* k_out, int64_t k_tok_stride,
+                                 uint16_t* v_out, int64_t v_tok_stride,
+                                 uint16_t* kt, uint16_t* vt, uintptr_t stream);
+
+/* pdk_rmsnorm_partials with split s at partials + s * split_stride elements (a
+ * multiple of 4), so that it can take some rows of a larger projection. */
+int pdk_prefill_rmsnorm_partials(uint16_t* x, const float* partials,
+                                 int64_t split_stride, int splits,
+                                 const uint16_t* weight, int B, int H, float eps,
+                                 uint16_t* out, uintptr_t stream);
+
 /* Causal GQA attention of the prompt: out [T][Hq][128] bf16 from q (rows of
  * q_tok_stride elements, Hq * 128 of them used) and pdk_prefill_rope_kv's kt
  * and vt. Query head h reads KV head h / (Hq / Hkv). Weights stay fp32. */

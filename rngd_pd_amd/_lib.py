@@ -136,6 +136,13 @@ SIGNATURES = {
     "pdk_rope_table": (_I, [_P, _I, _I, _P, _U]),
     "pdk_prefill_kv_tile_elems": (_I64, [_I, _I]),
     "pdk_prefill_rope_kv": (_I, [_P, _P, _I, _I, _I, _I, _P, _I64, _P, _I64, _P, _P, _U]),
+    "pdk_prefill_gemm_splits": (_I, [_I, _I, _I]),
+    "pdk_prefill_gemm": (_I, [_P, _P, _I, _I, _I, _P, _U]),
+    "pdk_prefill_gemm_swiglu_takes": (_I, [_I, _I, _I]),
+    "pdk_prefill_gemm_swiglu": (_I, [_P, _P, _I, _I, _I, _P, _U]),
+    "pdk_prefill_rope_kv_partials": (_I, [_P, _I, _P, _I, _I, _I, _I, _P, _P, _I64, _P, _I64, _P,
+                                          _P, _U]),
+    "pdk_prefill_rmsnorm_partials": (_I, [_P, _P, _I64, _I, _P, _I, _I, _F, _P, _U]),
     "pdk_prefill_attn": (_I, [_P, _I64, _P, _P, _I, _I, _I, _I, _F, _P, _U]),
     "pdk_scatter_koni": (_I, [_P, _I64, _P, _I, _I, _P, _I, _P, _P, _I64, _I, _I, _I, _U]),
     "pdk_host_alloc": (_I, [_SZ, ctypes.POINTER(_P)]),

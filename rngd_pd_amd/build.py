@@ -7,7 +7,7 @@ import sys
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _ROOT = os.path.dirname(_HERE)
 SOURCES = ["handoff.hip", "attention.hip", "decode_step.hip", "wgemm.hip",
-           "wgemm_wide.hip", "prefill.hip", "koni.hip", "staging.hip",
+           "wgemm_wide.hip", "prefill.hip", "prefill_gemm.hip", "koni.hip", "staging.hip",
            "runtime.hip"]
 OUT = os.path.join(_HERE, "librngdpd.so")
 NET_SOURCES = ["net/tcpkv.cpp"]
@@ -33,7 +33,8 @@ def hipcc_command(out=OUT):
 # column groups do spill and are allowed (wgemm_kernel is not listed).
 NO_SCRATCH = ("decode_attn_kernel", "merge_kernel", "pack_kernel", "scatter_kernel",
               "gather_kernel", "koni_scatter_kernel", "koni_gather_kernel",
-              "rope_kv_kernel", "prefill_attn_kernel", "wgemm_wide_kernel")
+              "rope_kv_kernel", "prefill_attn_kernel", "prefill_gemm_kernel",
+              "wgemm_wide_kernel")
 
 
 def resource_report(text):

@@ -30,13 +30,17 @@ __device__ __forceinline__ float wave_sum(float x) {
 // summed in a fixed order), written back. Then
 // out = bf16(x * rsqrt(mean(x^2) + eps) * w) (rms_dsl: x * (sum x^2 + eps*H)^-1/2
 // * w*sqrt(H), the same value).
-constexpr int kNormThreads = 256, kNormChunks = 4;     // 8 elements per chunk
+// The prefill's partials (up to 8 splits of a few rows) take 512 threads: each
+// row is then one chunk per thread at H = 4096, and 4 splits' loads are in
+// flight together (splits come one after another otherwise, a round trip each).
+constexpr int kNormThreads = 256, kNormMaxH = 8192;
 
-template <int kAdd>
-__global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(uint16_t* x, const void* add,
-                                                               int splits, int B,
-                                                               const uint16_t* w, float eps,
-                                                               int H, uint16_t* out) {
+template <int kAdd, int kThreads = kNormThreads>
+__global__ __launch_bounds__(kThreads) void rmsnorm_kernel(uint16_t* x, const void* add,
+                                                           int splits, int64_t split_stride,
+                                                           const uint16_t* w, float eps, int H,
+                                                           uint16_t* out) {
+  constexpr int kNormThreads = kThreads, kNormChunks = 1024 / kThreads;  // 8 elements per chunk
   __shared__ float part[kNormThreads / 64];
   const int64_t row = (int64_t)blockIdx.x * H;
   const int n8 = H >> 3;
@@ -68,11 +72,20 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(uint16_t* x, cons
 #pragma unroll
         for (int k = 0; k < 8; ++k) acc[k] = 0.f;
         const float* p = static_cast<const float*>(add) + row + 8 * c;
-        for (int s = 0; s < splits; ++s) {
-          const float4 u = *reinterpret_cast<const float4*>(p + (int64_t)s * B * H);
-          const float4 v = *reinterpret_cast<const float4*>(p + (int64_t)s * B * H + 4);
-          acc[0] += u.x; acc[1] += u.y; acc[2] += u.z; acc[3] += u.w;
-          acc[4] += v.x; acc[5] += v.y; acc[6] += v.z; acc[7] += v.w;
+        for (int s0 = 0; s0 < splits; s0 += 4) {
+          float4 u[4], v[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float* q = p + min(s0 + i, splits - 1) * split_stride;
+            u[i] = *reinterpret_cast<const float4*>(q);
+            v[i] = *reinterpret_cast<const float4*>(q + 4);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if (s0 + i >= splits) break;
+            acc[0] += u[i].x; acc[1] += u[i].y; acc[2] += u[i].z; acc[3] += u[i].w;
+            acc[4] += v[i].x; acc[5] += v[i].y; acc[6] += v[i].z; acc[7] += v[i].w;
+          }
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -309,8 +322,8 @@ extern "C" int pdk_embed_ssq_xt(const uint16_t* table, int64_t vocab, const void
 static int check_norm(const void* x, const void* weight, const void* out, int B, int H) {
   PDK_REQUIRE(x && weight && out, "null pointer argument");
   PDK_REQUIRE(B >= 1 && B <= 65535, "B must be in [1, 65535] (got %d)", B);
-  PDK_REQUIRE(H >= 8 && H % 8 == 0 && H <= kNormThreads * kNormChunks * 8,
-              "H must be a multiple of 8 in [8, %d] (got %d)", kNormThreads * kNormChunks * 8, H);
+  PDK_REQUIRE(H >= 8 && H % 8 == 0 && H <= kNormMaxH,
+              "H must be a multiple of 8 in [8, %d] (got %d)", kNormMaxH, H);
   PDK_REQUIRE(pdk::aligned16(x) && pdk::aligned16(weight) && pdk::aligned16(out),
               "tensors must be 16-byte aligned");
   return PDK_OK;
@@ -324,10 +337,10 @@ extern "C" int pdk_rmsnorm(uint16_t* x, const uint16_t* add, const uint16_t* wei
   PDK_REQUIRE(eps >= 0.f, "eps must be >= 0");
   hipStream_t st = pdk::as_stream(stream);
   if (add)
-    hipLaunchKernelGGL(rmsnorm_kernel<1>, dim3(B), dim3(kNormThreads), 0, st, x, add, 0, B,
+    hipLaunchKernelGGL(rmsnorm_kernel<1>, dim3(B), dim3(kNormThreads), 0, st, x, add, 0, 0,
                        weight, eps, H, out);
   else
-    hipLaunchKernelGGL(rmsnorm_kernel<0>, dim3(B), dim3(kNormThreads), 0, st, x, nullptr, 0, B,
+    hipLaunchKernelGGL(rmsnorm_kernel<0>, dim3(B), dim3(kNormThreads), 0, st, x, nullptr, 0, 0,
                        weight, eps, H, out);
   return pdk::check_launch("rmsnorm_kernel");
 }
@@ -341,7 +354,23 @@ extern "C" int pdk_rmsnorm_partials(uint16_t* x, const float* partials, int spli
   PDK_REQUIRE(splits >= 1 && splits <= 64, "splits must be in [1, 64] (got %d)", splits);
   PDK_REQUIRE(eps >= 0.f, "eps must be >= 0");
   hipLaunchKernelGGL(rmsnorm_kernel<2>, dim3(B), dim3(kNormThreads), 0, pdk::as_stream(stream),
-                     x, partials, splits, B, weight, eps, H, out);
+                     x, partials, splits, (int64_t)B * H, weight, eps, H, out);
+  return pdk::check_launch("rmsnorm_kernel");
+}
+
+extern "C" int pdk_prefill_rmsnorm_partials(uint16_t* x, const float* partials,
+                                            int64_t split_stride, int splits,
+                                            const uint16_t* weight, int B, int H, float eps,
+                                            uint16_t* out, uintptr_t stream) {
+  pdk::clear_error();
+  if (int rc = check_norm(x, weight, out, B, H)) return rc;
+  PDK_REQUIRE(partials && pdk::aligned16(partials), "partials must be 16-byte aligned");
+  PDK_REQUIRE(splits >= 1 && splits <= 64, "splits must be in [1, 64] (got %d)", splits);
+  PDK_REQUIRE(split_stride >= (int64_t)B * H && split_stride % 4 == 0,
+              "the split stride must be a multiple of 4 and hold B * H elements");
+  PDK_REQUIRE(eps >= 0.f, "eps must be >= 0");
+  hipLaunchKernelGGL((rmsnorm_kernel<2, 512>), dim3(B), dim3(512), 0, pdk::as_stream(stream), x,
+                     partials, splits, split_stride, weight, eps, H, out);
   return pdk::check_launch("rmsnorm_kernel");
 }
 

@@ -65,18 +65,52 @@ __global__ __launch_bounds__(256) void rope_table_kernel(const float* inv_freq, 
   table[idx] = make_float2(c, s);
 }
 
+// Eight elements of `splits` partial rows, added in order and rounded to bf16.
+__device__ __forceinline__ v8 partial_sum(const float* p, int splits, int64_t stride) {
+  float s[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) s[k] = 0.f;
+  for (int s0 = 0; s0 < splits; s0 += 4) {          // four splits' loads in flight
+    float4 u[4], v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float* q = p + min(s0 + i, splits - 1) * stride;
+      u[i] = *reinterpret_cast<const float4*>(q);
+      v[i] = *reinterpret_cast<const float4*>(q + 4);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (s0 + i >= splits) break;
+      s[0] += u[i].x; s[1] += u[i].y; s[2] += u[i].z; s[3] += u[i].w;
+      s[4] += v[i].x; s[5] += v[i].y; s[6] += v[i].z; s[7] += v[i].w;
+    }
+  }
+  v8 r;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) r.w[w] = pdk::pack_bf16x2_rne(s[2 * w], s[2 * w + 1]);
+  return r;
+}
+
 // One workgroup: a 32-token tile of kRopeHeads consecutive heads (of NH q, NKV
 // k, NKV v). Thread (r, o) = (tid / 8, tid % 8) holds token r, dims 8o..8o+7
 // and 64+8o..+7 (a rotation pair per element), and its 8 (cos, sin) pairs stay
 // in registers for all the heads: reading them per head would move as many
 // bytes as the heads themselves. Bound by the bytes of q|k|v in and out.
+//
+// kPart: q|k|v comes as `splits` fp32 partial sums [s][T][(NH + 2 NKV) 128]
+// (pdk_prefill_gemm's), added in order and rounded to bf16 once, and q goes to
+// rows of its own. Those are prompts of at most a few tiles: one head per
+// workgroup, so that more than 12 workgroups per tile share the reads.
 constexpr int kRopeHeads = 4;
 constexpr int kVRow = kD + 2;             // LDS row of the V transpose
 
-__global__ __launch_bounds__(256) void rope_kv_kernel(uint16_t* qkv, const float2* table, int T,
-                                                      int NH, int NKV, uint16_t* k_out,
-                                                      int64_t k_ld, uint16_t* v_out, int64_t v_ld,
-                                                      uint16_t* kt, uint16_t* vt) {
+template <bool kPart>
+__global__ __launch_bounds__(256) void rope_kv_kernel(uint16_t* qkv, const float* part, int splits,
+                                                      const float2* table, int T, int NH, int NKV,
+                                                      uint16_t* k_out, int64_t k_ld,
+                                                      uint16_t* v_out, int64_t v_ld, uint16_t* kt,
+                                                      uint16_t* vt) {
+  constexpr int kRopeHeads = kPart ? 1 : ::kRopeHeads;
   __shared__ uint16_t vs[kTile][kVRow];
   const int tile = blockIdx.x, n_tiles = gridDim.x;
   const int r = threadIdx.x >> 3, o = threadIdx.x & 7;
@@ -94,14 +128,20 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(uint16_t* qkv, const float
     }
   }
   const int n_heads = NH + 2 * NKV;
-  uint16_t* row = qkv + (int64_t)tc * n_heads * kD + 8 * o;
+  uint16_t* row = qkv + (int64_t)tc * (kPart ? NH : n_heads) * kD + 8 * o;
   const int h0 = blockIdx.y * kRopeHeads;
   v8 a[kRopeHeads], b[kRopeHeads];
 #pragma unroll
   for (int i = 0; i < kRopeHeads; ++i) {
     const int hd = min(h0 + i, n_heads - 1);
-    a[i] = pdk::ld16(row + (int64_t)hd * kD);
-    b[i] = pdk::ld16(row + (int64_t)hd * kD + kD / 2);
+    if constexpr (kPart) {
+      const float* p = part + ((int64_t)tc * n_heads + hd) * kD + 8 * o;
+      a[i] = partial_sum(p, splits, (int64_t)T * n_heads * kD);
+      b[i] = partial_sum(p + kD / 2, splits, (int64_t)T * n_heads * kD);
+    } else {
+      a[i] = pdk::ld16(row + (int64_t)hd * kD);
+      b[i] = pdk::ld16(row + (int64_t)hd * kD + kD / 2);
+    }
   }
 #pragma unroll
   for (int i = 0; i < kRopeHeads; ++i) {
@@ -358,10 +398,12 @@ extern "C" int64_t pdk_prefill_kv_tile_elems(int T, int n_kv_heads) {
   return (int64_t)n_kv_heads * ((T + kTile - 1) / kTile) * kTileElems;
 }
 
-extern "C" int pdk_prefill_rope_kv(uint16_t* qkv, const float* table, int T, int n_q_heads,
-                                   int n_kv_heads, int head_dim, uint16_t* k_out,
-                                   int64_t k_tok_stride, uint16_t* v_out, int64_t v_tok_stride,
-                                   uint16_t* kt, uint16_t* vt, uintptr_t stream) {
+namespace {
+
+template <bool kPart>
+int rope_kv(uint16_t* qkv, const float* part, int splits, const float* table, int T,
+            int n_q_heads, int n_kv_heads, int head_dim, uint16_t* k_out, int64_t k_tok_stride,
+            uint16_t* v_out, int64_t v_tok_stride, uint16_t* kt, uint16_t* vt, uintptr_t stream) {
   pdk::clear_error();
   if (head_dim != kD) {
     pdk::set_error("the prefill kernels implement head_dim %d only (got %d)", kD, head_dim);
@@ -375,12 +417,34 @@ extern "C" int pdk_prefill_rope_kv(uint16_t* qkv, const float* table, int T, int
   PDK_REQUIRE(k_tok_stride >= (int64_t)n_kv_heads * kD && k_tok_stride % 8 == 0 &&
                   v_tok_stride >= (int64_t)n_kv_heads * kD && v_tok_stride % 8 == 0,
               "token strides must be multiples of 8 and hold Hkv * D elements");
-  const dim3 grid((T + kTile - 1) / kTile,
-                  (n_q_heads + 2 * n_kv_heads + kRopeHeads - 1) / kRopeHeads);
-  hipLaunchKernelGGL(rope_kv_kernel, grid, dim3(256), 0, pdk::as_stream(stream), qkv,
-                     reinterpret_cast<const float2*>(table), T, n_q_heads, n_kv_heads, k_out,
-                     k_tok_stride, v_out, v_tok_stride, kt, vt);
+  PDK_REQUIRE(!kPart || (part && pdk::aligned16(part)), "partials must be 16-byte aligned");
+  PDK_REQUIRE(!kPart || (splits >= 1 && splits <= 64), "splits must be in [1, 64] (got %d)",
+              splits);
+  const int heads = kPart ? 1 : kRopeHeads;
+  const dim3 grid((T + kTile - 1) / kTile, (n_q_heads + 2 * n_kv_heads + heads - 1) / heads);
+  hipLaunchKernelGGL(rope_kv_kernel<kPart>, grid, dim3(256), 0, pdk::as_stream(stream), qkv, part,
+                     splits, reinterpret_cast<const float2*>(table), T, n_q_heads, n_kv_heads,
+                     k_out, k_tok_stride, v_out, v_tok_stride, kt, vt);
   return pdk::check_launch("rope_kv_kernel");
+}
+
+}  // namespace
+
+extern "C" int pdk_prefill_rope_kv(uint16_t* qkv, const float* table, int T, int n_q_heads,
+                                   int n_kv_heads, int head_dim, uint16_t* k_out,
+                                   int64_t k_tok_stride, uint16_t* v_out, int64_t v_tok_stride,
+                                   uint16_t* kt, uint16_t* vt, uintptr_t stream) {
+  return rope_kv<false>(qkv, nullptr, 0, table, T, n_q_heads, n_kv_heads, head_dim, k_out,
+                        k_tok_stride, v_out, v_tok_stride, kt, vt, stream);
+}
+
+extern "C" int pdk_prefill_rope_kv_partials(const float* partials, int splits, const float* table,
+                                            int T, int n_q_heads, int n_kv_heads, int head_dim,
+                                            uint16_t* q_out, uint16_t* k_out, int64_t k_tok_stride,
+                                            uint16_t* v_out, int64_t v_tok_stride, uint16_t* kt,
+                                            uint16_t* vt, uintptr_t stream) {
+  return rope_kv<true>(q_out, partials, splits, table, T, n_q_heads, n_kv_heads, head_dim, k_out,
+                       k_tok_stride, v_out, v_tok_stride, kt, vt, stream);
 }
 
 extern "C" int pdk_prefill_attn(const uint16_t* q, int64_t q_tok_stride, const uint16_t* kt,

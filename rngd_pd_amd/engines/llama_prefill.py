@@ -8,19 +8,21 @@ token of the last position (the reference's "next", serving/cluster.py:
 done, so saves overlap the layers that follow (the reference emits layer
 groups as it goes).
 
-Prefill is compute-bound (T tokens per weight), so its GEMMs are the
-library's (hipBLASLt through torch). Between them, at head_dim 128, one launch
-per line of a layer:
+Up to 256 tokens the GEMMs are pdk_prefill_gemm's (K split over workgroups, fp32
+partial sums that the next kernel adds up), the O and down projections' up to
+512; a longer prompt is compute-bound on tiles enough for every CU and its GEMMs
+are the library's (hipBLASLt through torch). At head_dim 128, one launch per line
+of a layer, the short prompt's on the right:
 
-  h = rmsnorm(x + down)                         pdk_rmsnorm, residual add fused
-  qkv = h . Wqkv^T                              library
-  RoPE; K/V rows; attention's operands          pdk_prefill_rope_kv
-  ao = causal GQA attention                     pdk_prefill_attn (fp32 weights)
-  o = ao . Wo^T                                 library
-  h = rmsnorm(x + o)                            pdk_rmsnorm, residual add fused
-  gu = h . Wgu^T                                library
-  act = silu(g) * u                             pdk_swiglu
-  down = act . Wd^T                             library
+  h = rmsnorm(x + down)                pdk_rmsnorm          pdk_prefill_rmsnorm_partials
+  qkv = h . Wqkv^T                     library              pdk_prefill_gemm
+  RoPE; K/V rows; attention's operands pdk_prefill_rope_kv  pdk_prefill_rope_kv_partials
+  ao = causal GQA attention            pdk_prefill_attn (fp32 weights)
+  o = ao . Wo^T                        library              pdk_prefill_gemm
+  h = rmsnorm(x + o)                   pdk_rmsnorm          pdk_prefill_rmsnorm_partials
+  gu = h . Wgu^T                       library              pdk_prefill_gemm_swiglu, with
+  act = silu(g) * u                    pdk_swiglu             this line
+  down = act . Wd^T                    library              pdk_prefill_gemm
 
 Other head dims take RoPE and attention as fp32 torch operations on contiguous
 operands. Activations are bf16 at tensor boundaries, as in the decode step. It
@@ -48,6 +50,55 @@ def _rows(t, shape, device):
     return ld if ld >= shape[1] * shape[2] and ld % 8 == 0 else None
 
 
+class _Partials:
+    """A projection as ``splits`` fp32 partial sums [splits, T, N], to be added by
+    the kernel that reads it."""
+
+    def __init__(self, buf, splits, T, N):
+        self.buf, self.splits, self.T, self.N = buf, splits, T, N
+
+
+class _Projections:
+    """The projections of one forward over T tokens. Those pdk_prefill_gemm takes
+    write their partial sums to one workspace: each is read by the launch after
+    it, before the next one writes."""
+
+    def __init__(self, cfg, T, device):
+        lib, H = _lib.lib(), cfg.hidden
+        self.T, self.device, self.M = T, device, cfg.inter
+        self.splits = {(N, K): lib.pdk_prefill_gemm_splits(T, K, N)
+                       for N, K in ((cfg.qkv_dim, H), (H, cfg.n_heads * cfg.head_dim),
+                                    (H, cfg.inter))}
+        self.fused = bool(lib.pdk_prefill_gemm_swiglu_takes(T, H, cfg.inter))
+        n = max(s * T * N for (N, _), s in self.splits.items())
+        self.buf = torch.empty(n, dtype=torch.float32, device=device) if n else None
+
+    def _direct(self, w):
+        """Whether a kernel can read this weight where it lies."""
+        return w.dtype == BF16 and w.device == self.device and w.is_contiguous() \
+            and w.data_ptr() % 16 == 0
+
+    def linear(self, x, w, partials=True):
+        """x . w^T: _Partials where the kernel takes the shape (and the caller
+        takes partials), else bf16."""
+        splits = self.splits.get(tuple(w.shape), 0) if partials else 0
+        if not splits or not self._direct(w):
+            return torch.nn.functional.linear(x, w)
+        N, K = w.shape
+        _lib.call("pdk_prefill_gemm", x.data_ptr(), w.data_ptr(), self.T, K, N,
+                  self.buf.data_ptr(), stream_handle())
+        return _Partials(self.buf, splits, self.T, N)
+
+    def swiglu(self, x, w):
+        """silu(x . wg^T) * (x . wu^T) in one launch, or None."""
+        if not self.fused or tuple(w.shape) != (2 * self.M, x.shape[1]) or not self._direct(w):
+            return None
+        act = torch.empty((self.T, self.M), dtype=BF16, device=self.device)
+        _lib.call("pdk_prefill_gemm_swiglu", x.data_ptr(), w.data_ptr(), self.T, x.shape[1],
+                  self.M, act.data_ptr(), stream_handle())
+        return act
+
+
 class LlamaPrefill:
     def __init__(self, weights, max_tokens=4096):
         self.w, self.cfg = weights, weights.cfg
@@ -57,8 +108,17 @@ class LlamaPrefill:
         self.inv = cfg.inv_freq().to(self.device)
         self.scale = 1.0 / math.sqrt(cfg.head_dim)
 
-    def _rmsnorm(self, x, weight, out, add=None):
-        """out = rmsnorm(x + add) * weight; with ``add``, x takes the sum."""
+    def _rmsnorm(self, x, weight, out, add=None, row=0):
+        """out = rmsnorm(x + add) * weight over the rows of x from ``row``; with
+        ``add``, x takes the sum."""
+        if isinstance(add, _Partials):
+            _lib.call("pdk_prefill_rmsnorm_partials", x[row:].data_ptr(),
+                      add.buf.data_ptr() + 4 * row * add.N, add.T * add.N, add.splits,
+                      weight.data_ptr(), add.T - row, add.N, self.cfg.eps, out.data_ptr(),
+                      stream_handle())
+            return out
+        if row:
+            x, add = x[row:], None if add is None else add[row:]
         T, H = x.shape
         _lib.call("pdk_rmsnorm", x.data_ptr(), None if add is None else add.data_ptr(),
                   weight.data_ptr(), T, H, self.cfg.eps, out.data_ptr(), stream_handle())
@@ -82,17 +142,27 @@ class LlamaPrefill:
         n = _lib.lib().pdk_prefill_kv_tile_elems(T, NKV)
         kt, vt = (torch.empty(n, dtype=BF16, device=dev) for _ in range(2))
         ao = torch.empty((T, NH * HD), dtype=BF16, device=dev)
+        q_rows = None
 
         def attention(qkv, k_l, v_l, before):
+            nonlocal q_rows
             rows = []
             for t in (k_l, v_l):
                 ld = _rows(t, (T, NKV, HD), dev)
                 own = t if ld else torch.empty((T, NKV, HD), dtype=BF16, device=dev)
                 rows.append((own, ld or NKV * HD))
             (k, k_ld), (v, v_ld) = rows
-            _lib.call("pdk_prefill_rope_kv", qkv.data_ptr(), table.data_ptr(), T, NH, NKV, HD,
-                      k.data_ptr(), k_ld, v.data_ptr(), v_ld, kt.data_ptr(), vt.data_ptr(),
-                      stream_handle())
+            outs = (k.data_ptr(), k_ld, v.data_ptr(), v_ld, kt.data_ptr(), vt.data_ptr(),
+                    stream_handle())
+            if isinstance(qkv, _Partials):
+                if q_rows is None:
+                    q_rows = torch.empty((T, NH * HD), dtype=BF16, device=dev)
+                _lib.call("pdk_prefill_rope_kv_partials", qkv.buf.data_ptr(), qkv.splits,
+                          table.data_ptr(), T, NH, NKV, HD, q_rows.data_ptr(), *outs)
+                qkv = q_rows
+            else:
+                _lib.call("pdk_prefill_rope_kv", qkv.data_ptr(), table.data_ptr(), T, NH, NKV, HD,
+                          *outs)
             if k is not k_l:
                 k_l.copy_(k)
             if v is not v_l:
@@ -156,8 +226,9 @@ class LlamaPrefill:
             v_all = torch.empty((L, T, NKV, HD), dtype=BF16, device=dev)
         else:
             k_all, v_all = kv_out
-        linear = torch.nn.functional.linear
-        attention = (self._kernel_attention if HD == 128 else self._torch_attention)(T)
+        fused = HD == 128
+        attention = (self._kernel_attention if fused else self._torch_attention)(T)
+        proj = _Projections(cfg, T, dev)
         x = w.embed.index_select(0, ids)                           # [T, H] bf16
         h = torch.empty_like(x)
         down = None                                                # not yet added to x
@@ -165,11 +236,14 @@ class LlamaPrefill:
             self._rmsnorm(x, w.norm1[li], h, add=down)
             k_l, v_l = k_all[li], v_all[li]
             emit = (lambda: None) if on_layer is None else (lambda: on_layer(li, k_l, v_l))
-            ao = attention(linear(h, w.wqkv[li]), k_l, v_l, emit)
-            self._rmsnorm(x, w.norm2[li], h, add=linear(ao, w.wo[li]))
-            down = linear(self._swiglu(linear(h, w.wgu[li])), w.wd[li])
+            ao = attention(proj.linear(h, w.wqkv[li], partials=fused), k_l, v_l, emit)
+            self._rmsnorm(x, w.norm2[li], h, add=proj.linear(ao, w.wo[li]))
+            act = proj.swiglu(h, w.wgu[li])
+            if act is None:
+                act = self._swiglu(torch.nn.functional.linear(h, w.wgu[li]))
+            down = proj.linear(act, w.wd[li])
         last = torch.empty((1, H), dtype=BF16, device=dev)
-        self._rmsnorm(x[T - 1:], w.norm_f, last, add=None if down is None else down[T - 1:])
-        logits = linear(last, w.lm_head)
+        self._rmsnorm(x, w.norm_f, last, add=down, row=T - 1)
+        logits = torch.nn.functional.linear(last, w.lm_head)
         first = int(torch.argmax(logits[0]).item())
         return first, k_all, v_all
