@@ -723,6 +723,14 @@ int pdk_prefill_rmsnorm_partials(uint16_t* x, const float* partials,
                                  const uint16_t* weight, int B, int H, float eps,
                                  uint16_t* out, uintptr_t stream);
 
+/* The greedy token of one row of logits given as partial sums [splits][1][N]
+ * (pdk_prefill_gemm's at T = 1): keys[i], i < ceil(N / 1024), is the best key of
+ * columns 1024 i .. (as pdk_linear_argmax's: the value in an order-preserving
+ * code above the complement of the column), so the token is 0xffffffff minus the
+ * low 32 bits of the largest. */
+int pdk_prefill_argmax(const float* partials, int splits, int N, uint64_t* keys,
+                       uintptr_t stream);
+
 /* Causal GQA attention of the prompt: out [T][Hq][128] bf16 from q (rows of
  * q_tok_stride elements, Hq * 128 of them used) and pdk_prefill_rope_kv's kt
  * and vt. Query head h reads KV head h / (Hq / Hkv). Weights stay fp32. */

@@ -143,6 +143,7 @@ SIGNATURES = {
     "pdk_prefill_rope_kv_partials": (_I, [_P, _I, _P, _I, _I, _I, _I, _P, _P, _I64, _P, _I64, _P,
                                           _P, _U]),
     "pdk_prefill_rmsnorm_partials": (_I, [_P, _P, _I64, _I, _P, _I, _I, _F, _P, _U]),
+    "pdk_prefill_argmax": (_I, [_P, _I, _I, _P, _U]),
     "pdk_prefill_attn": (_I, [_P, _I64, _P, _P, _I, _I, _I, _I, _F, _P, _U]),
     "pdk_scatter_koni": (_I, [_P, _I64, _P, _I, _I, _P, _I, _P, _P, _I64, _I, _I, _I, _U]),
     "pdk_host_alloc": (_I, [_SZ, ctypes.POINTER(_P)]),

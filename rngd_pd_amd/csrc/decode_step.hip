@@ -31,8 +31,8 @@ __device__ __forceinline__ float wave_sum(float x) {
 // out = bf16(x * rsqrt(mean(x^2) + eps) * w) (rms_dsl: x * (sum x^2 + eps*H)^-1/2
 // * w*sqrt(H), the same value).
 // The prefill's partials (up to 8 splits of a few rows) take 512 threads: each
-// row is then one chunk per thread at H = 4096, and 4 splits' loads are in
-// flight together (splits come one after another otherwise, a round trip each).
+// row is then one chunk per thread at H = 4096, with all its splits' loads in
+// flight together (one after another they cost a round trip each).
 constexpr int kNormThreads = 256, kNormMaxH = 8192;
 
 template <int kAdd, int kThreads = kNormThreads>
@@ -41,6 +41,7 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_kernel(uint16_t* x, const vo
                                                            const uint16_t* w, float eps, int H,
                                                            uint16_t* out) {
   constexpr int kNormThreads = kThreads, kNormChunks = 1024 / kThreads;  // 8 elements per chunk
+  constexpr int kFlight = kThreads > 256 ? 8 : 2;
   __shared__ float part[kNormThreads / 64];
   const int64_t row = (int64_t)blockIdx.x * H;
   const int n8 = H >> 3;
@@ -72,16 +73,16 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_kernel(uint16_t* x, const vo
 #pragma unroll
         for (int k = 0; k < 8; ++k) acc[k] = 0.f;
         const float* p = static_cast<const float*>(add) + row + 8 * c;
-        for (int s0 = 0; s0 < splits; s0 += 4) {
-          float4 u[4], v[4];
+        for (int s0 = 0; s0 < splits; s0 += kFlight) {
+          float4 u[kFlight], v[kFlight];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
+          for (int i = 0; i < kFlight; ++i) {
             const float* q = p + min(s0 + i, splits - 1) * split_stride;
             u[i] = *reinterpret_cast<const float4*>(q);
             v[i] = *reinterpret_cast<const float4*>(q + 4);
           }
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
+          for (int i = 0; i < kFlight; ++i) {
             if (s0 + i >= splits) break;
             acc[0] += u[i].x; acc[1] += u[i].y; acc[2] += u[i].z; acc[3] += u[i].w;
             acc[4] += v[i].x; acc[5] += v[i].y; acc[6] += v[i].z; acc[7] += v[i].w;

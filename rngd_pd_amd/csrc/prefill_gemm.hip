@@ -15,9 +15,16 @@
 // buffer is refilled next.
 //
 // LDS rows are 64 columns (128 bytes, eight 16-byte chunks); chunk c of row r
-// holds columns 8 (c ^ (r & 7)) .., so the 16 rows a fragment read touches spread
-// over the banks. global_load_lds writes LDS in lane order, so the swizzle is
-// applied to the addresses the lanes load from.
+// holds columns 8 (c ^ (r / 2 & 7)) .., so that each group of 16 lanes that a
+// ds_read_b128 serves in one cycle touches all 64 banks: no conflicts counted,
+// where c ^ (r & 7) has as many conflict cycles as useful ones. global_load_lds
+// writes LDS in lane order, so the swizzle is applied to the addresses the lanes
+// load from.
+//
+// With no K split or two (gate|up, the lm_head) the workgroups would read the same columns at a
+// time, rows 8 KiB apart, which the memory channels serve unevenly: each column
+// tile starts 8 stages after its neighbour and wraps around (41 tokens 46.4 ->
+// 42.1 us, 1 token 44.0 -> 42.0, 100 tokens 49.5 -> 47.3).
 //
 // W is the A operand and X the B operand of v_mfma_f32_16x16x32_bf16: a lane
 // then holds four consecutive output columns of one token.
@@ -28,7 +35,7 @@
 //   q|k|v   4096 -> 6144  [8]  14.5 -> 10.4 17.7 -> 11.9 25.6 -> 16.0
 //   O       4096 -> 4096  [6]  15.5 ->  8.0 13.7 ->  9.3 24.4 -> 13   28.7 -> 24.1
 //   down   14336 -> 4096 [20]  26.5 -> 21.2 39.4 -> 22.8 75.4 -> 29.4 93.0 -> 64.3
-//   gate|up 4096 -> 28672 [39] 57.0 -> 43.8 48.5 -> 44.4 55.1 -> 52.4
+//   gate|up 4096 -> 28672 [39] 57.0 -> 42.0 48.5 -> 42.1 55.1 -> 50
 // (gate|up with its SwiGLU, which is a launch of its own after the library's).
 #include <math.h>
 
@@ -98,7 +105,7 @@ __global__ __launch_bounds__(64 * WM * WN, kMinWaves) void prefill_gemm_kernel(
     if (at >= BN / 8) p = x + (int64_t)min(m0 + r - BN, T - 1) * K;
     else if (kGlu && r >= BC) p = w + (int64_t)(N + min(n0 + r - BC, N - 1)) * K;
     else p = w + (int64_t)min(n0 + r, N - 1) * K;
-    src[i] = p + (int64_t)first * kBK + ((lane & 7) ^ (r & 7)) * 8;
+    src[i] = p + (int64_t)first * kBK + ((lane & 7) ^ ((r >> 1) & 7)) * 8;
     dst[i] = at * 512;
   }
   f32x4 acc[FN][FM];
@@ -107,18 +114,20 @@ __global__ __launch_bounds__(64 * WM * WN, kMinWaves) void prefill_gemm_kernel(
 #pragma unroll
     for (int b = 0; b < FM; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
   // A fragment's lane reads row lane % 16, columns 32 kc + 8 (lane / 16) .. + 7.
-  const int frag = (lane & 15) * kBK + ((lane >> 4) ^ (lane & 7)) * 8;
+  const int frag = (lane & 15) * kBK + ((lane >> 4) ^ ((lane >> 1) & 7)) * 8;
   int row[FN];                                         // first W row of fragment a
 #pragma unroll
   for (int a = 0; a < FN; ++a)
     row[a] = kGlu ? (a < FN / 2 ? 0 : BC) + wn * (BC / WN) + a % (FN / 2) * 16
                   : wn * (BN / WN) + a * 16;
 
-  auto issue = [&](uint16_t* __restrict__ to, int step) __attribute__((always_inline)) {
+  const int rot = splits <= 2 ? n0 / BC * 8 % n : 0;
+  auto issue = [&](uint16_t* __restrict__ to, int i) __attribute__((always_inline)) {
+    const int step = i + rot - (i + rot >= n ? n : 0);
 #pragma unroll
-    for (int i = 0; i < L; ++i)
-      __builtin_amdgcn_global_load_lds((global_void*)(src[i] + (int64_t)step * kBK),
-                                       (lds_void*)(to + dst[i]), 16, 0, 0);
+    for (int l = 0; l < L; ++l)
+      __builtin_amdgcn_global_load_lds((global_void*)(src[l] + (int64_t)step * kBK),
+                                       (lds_void*)(to + dst[l]), 16, 0, 0);
   };
   auto products = [&](const uint16_t* __restrict__ from) __attribute__((always_inline)) {
 #pragma unroll
@@ -185,6 +194,27 @@ __global__ __launch_bounds__(64 * WM * WN, kMinWaves) void prefill_gemm_kernel(
       }
     }
   }
+}
+
+// The best wg::argmax_key of 1024 columns of one row of partial sums, added in
+// order and rounded to bf16 (the logit), per workgroup.
+__global__ __launch_bounds__(256) void prefill_argmax_kernel(const float* part, int splits, int N,
+                                                             uint64_t* keys) {
+  __shared__ uint64_t best[4];
+  const int c = (blockIdx.x * 256 + threadIdx.x) * 4;
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+  const int at = min(c, N - 4);                        // N % 4 == 0
+  for (int s = 0; s < splits; ++s)
+    sum += *reinterpret_cast<const f32x4*>(part + (int64_t)s * N + at);
+  uint64_t key = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (c < N) key = max(key, argmax_key(pdk::pack_bf16x2_rne(sum[e], 0.f), c + e));
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) key = max(key, (uint64_t)__shfl_xor((unsigned long long)key, o));
+  if ((threadIdx.x & 63) == 0) best[threadIdx.x >> 6] = key;
+  __syncthreads();
+  if (threadIdx.x == 0) keys[blockIdx.x] = max(max(best[0], best[1]), max(best[2], best[3]));
 }
 
 // Tiles by the number of tokens. At most 64 of them leave the kernel bound by
@@ -273,4 +303,17 @@ extern "C" int pdk_prefill_gemm_swiglu(const uint16_t* x, const uint16_t* w_gate
   PDK_REQUIRE(pdk_prefill_gemm_swiglu_takes(T, K, M), "T=%d K=%d M=%d is not a shape this GEMM takes",
               T, K, M);
   return launch<true>(x, w_gate_up, T, K, M, 1, y, pdk::as_stream(stream));
+}
+
+extern "C" int pdk_prefill_argmax(const float* partials, int splits, int N, uint64_t* keys,
+                                  uintptr_t stream) {
+  pdk::clear_error();
+  PDK_REQUIRE(partials && keys, "null pointer argument");
+  PDK_REQUIRE(pdk::aligned16(partials) && ((uintptr_t)keys & 7u) == 0,
+              "partials must be 16-byte aligned and keys 8-byte aligned");
+  PDK_REQUIRE(N >= 4 && N % 4 == 0, "N must be a positive multiple of 4 (got %d)", N);
+  PDK_REQUIRE(splits >= 1 && splits <= 64, "splits must be in [1, 64] (got %d)", splits);
+  hipLaunchKernelGGL(prefill_argmax_kernel, dim3((N + 1023) / 1024), dim3(256), 0,
+                     pdk::as_stream(stream), partials, splits, N, keys);
+  return pdk::check_launch("prefill_argmax_kernel");
 }

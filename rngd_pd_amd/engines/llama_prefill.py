@@ -73,7 +73,7 @@ class _Projections:
         n = max(s * T * N for (N, _), s in self.splits.items())
         self.buf = torch.empty(n, dtype=torch.float32, device=device) if n else None
 
-    def _direct(self, w):
+    def direct(self, w):
         """Whether a kernel can read this weight where it lies."""
         return w.dtype == BF16 and w.device == self.device and w.is_contiguous() \
             and w.data_ptr() % 16 == 0
@@ -82,7 +82,7 @@ class _Projections:
         """x . w^T: _Partials where the kernel takes the shape (and the caller
         takes partials), else bf16."""
         splits = self.splits.get(tuple(w.shape), 0) if partials else 0
-        if not splits or not self._direct(w):
+        if not splits or not self.direct(w):
             return torch.nn.functional.linear(x, w)
         N, K = w.shape
         _lib.call("pdk_prefill_gemm", x.data_ptr(), w.data_ptr(), self.T, K, N,
@@ -91,7 +91,7 @@ class _Projections:
 
     def swiglu(self, x, w):
         """silu(x . wg^T) * (x . wu^T) in one launch, or None."""
-        if not self.fused or tuple(w.shape) != (2 * self.M, x.shape[1]) or not self._direct(w):
+        if not self.fused or tuple(w.shape) != (2 * self.M, x.shape[1]) or not self.direct(w):
             return None
         act = torch.empty((self.T, self.M), dtype=BF16, device=self.device)
         _lib.call("pdk_prefill_gemm_swiglu", x.data_ptr(), w.data_ptr(), self.T, x.shape[1],
@@ -210,6 +210,22 @@ class LlamaPrefill:
         _lib.call("pdk_swiglu", gu.data_ptr(), T, M, act.data_ptr(), stream_handle())
         return act
 
+    def _greedy(self, last, lm_head, proj):
+        """The token of the largest logit of last [1, H] (the first of equals). The
+        head is one row of the short prompts' GEMM; the host takes the largest of
+        the few keys that the partial sums reduce to."""
+        N, K = lm_head.shape
+        splits = _lib.lib().pdk_prefill_gemm_splits(1, K, N) if proj.direct(lm_head) else 0
+        if not splits:
+            return int(torch.argmax(torch.nn.functional.linear(last, lm_head)[0]).item())
+        part = torch.empty(splits * N, dtype=torch.float32, device=self.device)
+        keys = torch.empty(-(-N // 1024), dtype=torch.int64, device=self.device)
+        st = stream_handle()
+        _lib.call("pdk_prefill_gemm", last.data_ptr(), lm_head.data_ptr(), 1, K, N,
+                  part.data_ptr(), st)
+        _lib.call("pdk_prefill_argmax", part.data_ptr(), splits, N, keys.data_ptr(), st)
+        return 0xffffffff - (max(keys.tolist()) & 0xffffffff)
+
     @torch.no_grad()
     def forward(self, tokens, on_layer=None, kv_out=None):
         """tokens: int sequence or int64 tensor [T] (T >= 1). Returns (first
@@ -244,6 +260,4 @@ class LlamaPrefill:
             down = proj.linear(act, w.wd[li])
         last = torch.empty((1, H), dtype=BF16, device=dev)
         self._rmsnorm(x, w.norm_f, last, add=down, row=T - 1)
-        logits = torch.nn.functional.linear(last, w.lm_head)
-        first = int(torch.argmax(logits[0]).item())
-        return first, k_all, v_all
+        return self._greedy(last, w.lm_head, proj), k_all, v_all

@@ -114,6 +114,23 @@ def test_norm_from_partials(cuda, T, H, splits, first):
     assert ((out.double() - want).abs() <= want.abs() * (2.0 ** -8 + H * 2.0 ** -25)).all()
 
 
+@pytest.mark.parametrize("N,splits", [(4, 1), (1020, 3), (1028, 2), (16032, 2)])
+def test_argmax_of_partials(cuda, N, splits):
+    part = torch.randn((splits, N), generator=torch.Generator().manual_seed(N)).to(cuda)
+    part[:, N // 2:] = part[:, :N - N // 2]                    # ties: the first counts
+    total = torch.zeros(N, device=cuda)
+    for p in part:
+        total = total + p
+    keys = torch.empty(-(-N // 1024), dtype=torch.int64, device=cuda)
+    for case in ("plain", "inf", "nan"):
+        if case != "plain":
+            part[0, N - 1] = total[N - 1] = float(case)
+        _lib.call("pdk_prefill_argmax", part.data_ptr(), splits, N, keys.data_ptr(),
+                  stream_handle())
+        got = 0xffffffff - (max(keys.tolist()) & 0xffffffff)
+        assert got == int(torch.argmax(total.to(BF16).float().cpu())), case
+
+
 def test_forward_on_both_sides_of_the_switches(cuda):
     """A prompt's first tokens have the same KV whatever kernels its length
     takes, and a weight the kernels cannot read takes the library."""
@@ -130,7 +147,8 @@ def test_forward_on_both_sides_of_the_switches(cuda):
     for weights, lengths in ((w, (1, 16, 17, 33, 65, 129, 256, 257, 512)), (odd, (40,))):
         for T in lengths:
             print(f"forward T={T}", flush=True)
-            _, a, b = LlamaPrefill(weights).forward(tokens[:T])
+            first, a, b = LlamaPrefill(weights).forward(tokens[:T])
+            assert 0 <= first < 300
             for got, want in ((a, k[:, :T]), (b, v[:, :T])):
                 # bf16 activations through three layers.
                 assert (got.float() - want.float()).norm() <= 1e-2 * want.float().norm()
