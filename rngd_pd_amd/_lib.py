@@ -214,5 +214,12 @@ def check(rc, what):
     raise PdkError(rc, what, last_error())
 
 
+_fns = {}
+
+
 def call(name, *args):
-    return check(getattr(lib(), name)(*args), name)
+    fn = _fns.get(name)
+    if fn is None:
+        fn = _fns[name] = getattr(lib(), name)
+    rc = fn(*args)
+    return rc if rc == PDK_OK else check(rc, name)

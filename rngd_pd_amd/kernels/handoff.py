@@ -25,7 +25,10 @@ BF16 = torch.bfloat16
 def stream_handle(stream=None):
     """hipStream_t of a torch stream (default: the current stream) as an int."""
     if stream is None:
-        return torch.cuda.current_stream().cuda_stream
+        if not torch.cuda.is_initialized():
+            return torch.cuda.current_stream().cuda_stream
+        # The same handle without a Stream object, which costs the host 2 us.
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
@@ -54,11 +57,12 @@ def _as_layers(k, v):
     if k.dim() != 4 or k.shape != v.shape:
         raise ValueError(f"k/v must be [L, T, Hkv, D] of equal shape, got {tuple(k.shape)} "
                          f"and {tuple(v.shape)}")
-    L, T, H, D = k.shape
-    for name, t in (("k", k), ("v", v)):
-        if t.stride(3) != 1 or t.stride(2) != D:
+    D = k.shape[3]
+    strides, other = k.stride(), v.stride()
+    for name, st in (("k", strides), ("v", other)):
+        if st[3] != 1 or st[2] != D:
             raise ValueError(f"{name}: [Hkv, D] must be contiguous per token")
-    if k.stride(0) != v.stride(0) or k.stride(1) != v.stride(1):
+    if strides[:2] != other[:2]:
         raise ValueError("k and v must share layer and token strides")
     return k, v
 
@@ -101,22 +105,25 @@ def pack_kv_batch(reqs, S, narrow=False, stream=None):
     leaves columns >= num_tokens unwritten (device-only consumers)."""
     if not reqs:
         return
-    L = H = D = None
+    L = H = D = want = None
     arr = []
     for k, v, P, frame in reqs:
         _need(k, "k")
         _need(v, "v")
         k, v = _as_layers(k, v)
+        l, T, h, d = k.shape
         if L is None:
-            L, _, H, D = k.shape
-        if (k.shape[0], k.shape[2], k.shape[3]) != (L, H, D):
+            L, H, D = l, h, d
+            want = frame_shape(L, H, D, S)
+        if (l, h, d) != (L, H, D):
             raise ValueError("all requests of a batch must share (L, Hkv, D)")
-        if not 0 <= P <= min(k.shape[1], S):
+        if not 0 <= P <= min(T, S):
             raise ValueError(f"num_tokens={P} outside [0, min(T, S)]")
-        if tuple(frame.shape) != frame_shape(L, H, D, S) or not frame.is_contiguous():
-            raise ValueError(f"frame must be contiguous {frame_shape(L, H, D, S)}")
-        arr.append(PackReq(k.data_ptr(), v.data_ptr(), frame.data_ptr(), k.stride(0),
-                           k.stride(1), int(P), _lib.PDK_PACK_NARROW if narrow else 0))
+        if frame.shape != want or not frame.is_contiguous():
+            raise ValueError(f"frame must be contiguous {want}")
+        strides = k.stride()
+        arr.append(PackReq(k.data_ptr(), v.data_ptr(), frame.data_ptr(), strides[0], strides[1],
+                           int(P), _lib.PDK_PACK_NARROW if narrow else 0))
     st = stream_handle(stream)
     for i in range(0, len(arr), PDK_MAX_BATCH):
         chunk = arr[i:i + PDK_MAX_BATCH]
@@ -130,7 +137,7 @@ def _check_cache(cache_k, cache_v):
     if cache_k.dim() == 4:
         cache_k, cache_v = cache_k.unsqueeze(0), cache_v.unsqueeze(0)
     L, nb, H, bs, D = cache_k.shape
-    if bs != PDK_BLOCK_SIZE or tuple(cache_v.shape) != (L, nb, H, D, bs):
+    if bs != PDK_BLOCK_SIZE or cache_v.shape != (L, nb, H, D, bs):
         raise ValueError(f"cache_k must be [L, nb, Hkv, 16, D] and cache_v [L, nb, Hkv, D, 16]; "
                          f"got {tuple(cache_k.shape)}, {tuple(cache_v.shape)}")
     if not (cache_k.is_contiguous() and cache_v.is_contiguous()):
@@ -187,11 +194,11 @@ def scatter_paged_batch(reqs, S, cache_k, cache_v, stream=None, skipped=None):
     that read and raises."""
     cache_k, cache_v = _check_cache(cache_k, cache_v)
     L, nb, H, _, D = cache_k.shape
-    arr = []
+    arr, want = [], frame_shape(L, H, D, S)
     for frame, table, P in reqs:
         _need(frame, "frame")
-        if tuple(frame.shape) != frame_shape(L, H, D, S) or not frame.is_contiguous():
-            raise ValueError(f"frame must be contiguous {frame_shape(L, H, D, S)}")
+        if frame.shape != want or not frame.is_contiguous():
+            raise ValueError(f"frame must be contiguous {want}")
         _need(table, "table", torch.int32)
         arr.append(ScatterReq(frame.data_ptr(), table.data_ptr(), int(P), table.numel()))
     if skipped is not None:
