@@ -21,10 +21,11 @@
 // writes LDS in lane order, so the swizzle is applied to the addresses the lanes
 // load from.
 //
-// With no K split or two (gate|up, the lm_head) the workgroups would read the same columns at a
-// time, rows 8 KiB apart, which the memory channels serve unevenly: each column
-// tile starts 8 stages after its neighbour and wraps around (41 tokens 46.4 ->
-// 42.1 us, 1 token 44.0 -> 42.0, 100 tokens 49.5 -> 47.3).
+// With one or two K splits (gate|up, the lm_head) the workgroups would read the
+// same columns at a time, rows 8 KiB apart, which the memory channels serve
+// unevenly: each column tile starts 8 stages after its neighbour and wraps around
+// (gate|up at 41 tokens 46.4 -> 42.1 us, 1 token 44.0 -> 42.0, 100 tokens 49.5 ->
+// 47.3; the lm_head of 16032 rows 30.9 -> 24.0).
 //
 // W is the A operand and X the B operand of v_mfma_f32_16x16x32_bf16: a lane
 // then holds four consecutive output columns of one token.
@@ -33,7 +34,7 @@
 // weights that do not fit the last-level cache; HBM alone at 6 TB/s in brackets):
 //   tokens                     1            41           128          470
 //   q|k|v   4096 -> 6144  [8]  14.5 -> 10.4 17.7 -> 11.9 25.6 -> 16.0
-//   O       4096 -> 4096  [6]  15.5 ->  8.0 13.7 ->  9.3 24.4 -> 13   28.7 -> 24.1
+//   O       4096 -> 4096  [6]  15.5 ->  7.4 13.7 ->  8.5 24.4 -> 11.7 28.7 -> 24.1
 //   down   14336 -> 4096 [20]  26.5 -> 21.2 39.4 -> 22.8 75.4 -> 29.4 93.0 -> 64.3
 //   gate|up 4096 -> 28672 [39] 57.0 -> 42.0 48.5 -> 42.1 55.1 -> 50
 // (gate|up with its SwiGLU, which is a launch of its own after the library's).
@@ -220,17 +221,27 @@ __global__ __launch_bounds__(256) void prefill_argmax_kernel(const float* part, 
 // Tiles by the number of tokens. At most 64 of them leave the kernel bound by
 // W, where 128 weight rows x 4 stages (64 KiB) per CU are in flight and more
 // rows of X would only take LDS; from 129 on two token tiles share each part of
-// W. Splits fill 256 CUs (two workgroups each for the 36 KiB tiles), at most 8
+// W. Without a K split (gate|up) the 64-column tiles of 17 to 32 tokens make a
+// nearly empty second wave: 51.3 us at 17 tokens in the model, 64 x 128 tiles
+// take 42.7.
+// Splits fill 256 CUs (two workgroups each for the 36 KiB tiles), at most 8
 // and each of at least 4 stages: one split more costs T * N * 8 bytes.
+//
+// narrow: where 128 columns would need those 8 splits of a short K (the O
+// projection: N and K 4096), 64 columns and 4 splits: O at 1 token 8.0 -> 7.4 us,
+// 24 8.5 -> 7.9, 41 9.6 -> 8.5, 100 12.2 -> 10.9, and half the partial sums to read.
+// The down projection (K 14336) has stages enough and gains nothing from it.
 struct Plan {
   int bm, bn, target;
+  bool narrow;
 };
-Plan plan_for(int T) {
-  if (T <= 16) return {16, 128, 256};
-  if (T <= 32) return {32, 64, 512};
-  if (T <= 64) return {64, 128, 256};
-  if (T <= 128) return {128, 128, 256};
-  return {128, 256, 256};
+Plan plan_for(int T, int K, int cols, bool glu) {
+  if (T > 128) return {128, 256, 256, false};
+  const bool narrow = !glu && K <= 4096 && (cols + 127) / 128 <= 32;
+  if (T <= 16) return {16, narrow ? 64 : 128, 256, narrow};
+  if (T <= 32 && !glu) return {32, 64, narrow ? 256 : 512, narrow};
+  if (T <= 64) return {64, narrow ? 64 : 128, 256, narrow};
+  return {128, narrow ? 64 : 128, 256, narrow};
 }
 int64_t tiles_of(const Plan& p, int T, int cols) {
   return (int64_t)((T + p.bm - 1) / p.bm) * ((cols + p.bn - 1) / p.bn);
@@ -242,11 +253,11 @@ int64_t tiles_of(const Plan& p, int T, int cols) {
 // gate|up 104 (with SwiGLU 115) and 120 of the best tile, 132 of these.
 bool takes(int T, int K, int rows) {
   if (T < 1 || K < 4 * kBK || K % kBK || rows < 4 || rows % 4) return false;
-  return T <= 256 || (T <= 512 && tiles_of(plan_for(T), T, rows) <= 64);
+  return T <= 256 || (T <= 512 && tiles_of(plan_for(T, K, rows, false), T, rows) <= 64);
 }
 
 int splits_for(int T, int K, int N) {
-  const Plan p = plan_for(T);
+  const Plan p = plan_for(T, K, N, false);
   const int64_t s = p.target / tiles_of(p, T, N);
   return (int)std::max<int64_t>(1, std::min<int64_t>({s, 8, K / kBK / 4}));
 }
@@ -254,15 +265,27 @@ int splits_for(int T, int K, int N) {
 template <bool kGlu>
 int launch(const uint16_t* x, const uint16_t* w, int T, int K, int N, int splits, void* out,
            hipStream_t st) {
-  const Plan p = plan_for(T);
+  const Plan p = plan_for(T, K, N, kGlu);
   const int m_tiles = (T + p.bm - 1) / p.bm;
   const int64_t blocks = tiles_of(p, T, kGlu ? 2 * N : N) * splits;
   PDK_REQUIRE(blocks < (1ll << 31), "launch too large");
 #define PDK_PG(BM, BN, WM, WN, S, OCC)                                                        \
   hipLaunchKernelGGL((prefill_gemm_kernel<BM, BN, WM, WN, S, kGlu, OCC>), dim3((unsigned)blocks), \
                      dim3(64 * WM * WN), 0, st, x, w, T, K, N, splits, m_tiles, out)
+  if constexpr (!kGlu) {                         // tiles gate|up never takes
+    if (p.narrow) {
+      if (T <= 16) PDK_PG(16, 64, 1, 4, 4, 2);
+      else if (T <= 32) PDK_PG(32, 64, 1, 4, 4, 2);
+      else if (T <= 64) PDK_PG(64, 64, 2, 2, 4, 2);
+      else PDK_PG(128, 64, 4, 2, 4, 1);
+      return pdk::check_launch("prefill_gemm_kernel");
+    }
+    if (p.bm == 32) {
+      PDK_PG(32, 64, 2, 2, 3, 4);
+      return pdk::check_launch("prefill_gemm_kernel");
+    }
+  }
   if (T <= 16) PDK_PG(16, 128, 1, 4, 4, 1);
-  else if (T <= 32) PDK_PG(32, 64, 2, 2, 3, 4);
   else if (T <= 64) PDK_PG(64, 128, 2, 4, 4, 1);
   else if (T <= 128) PDK_PG(128, 128, 2, 4, 4, 2);
   else PDK_PG(128, 256, 2, 4, 3, 2);

@@ -20,7 +20,9 @@ def _rand(seed, *shape, std=1.0):
     (1, 256, 4), (1, 4096, 512), (15, 320, 132), (16, 1024, 128), (17, 256, 64), (31, 2112, 68),
     (32, 704, 60), (33, 256, 260), (64, 1088, 124), (65, 256, 128), (128, 960, 132),
     (129, 256, 252), (200, 4096, 256), (256, 320, 516), (257, 512, 4), (385, 1024, 260),
-    (512, 14336, 256)])
+    (512, 14336, 256),
+    # more than 32 tiles of 128 columns, or a K above 4096: the wider tiles
+    (16, 256, 4100), (32, 320, 4100), (64, 4160, 100), (63, 256, 4228), (128, 4160, 132)])
 def test_partials(cuda, T, K, N):
     s = _lib.lib().pdk_prefill_gemm_splits(T, K, N)
     print(f"prefill gemm T={T} K={K} N={N} splits={s}", flush=True)
