@@ -200,10 +200,14 @@ int pdk_decode_attn(const uint16_t* q, const uint16_t* cache_k,
                     void* workspace, size_t workspace_bytes, uint16_t* out,
                     uintptr_t stream);
 
-/* pdk_cache_append followed by pdk_decode_attn, in one launch and with the
- * same results, bit for bit: the new token's k_new and v_new [B][n_kv_heads]
- * [head_dim] (16-byte aligned) go to slot ctx_lens[b] - 1 of the cache and
- * take part in the attention. No two streams may share that slot's block. */
+/* pdk_cache_append followed by pdk_decode_attn with the same results, bit for
+ * bit: the new token's k_new and v_new [B][n_kv_heads][head_dim] (16-byte
+ * aligned) go to slot ctx_lens[b] - 1 of the cache and take part in the
+ * attention, also in that of other streams whose tables hold the slot's block.
+ * Two streams with one and the same slot leave either's token there, and each
+ * attends over its own. One launch for up to 64 streams; two for more, for more
+ * than 256 (stream, KV head) pairs at contexts where two are faster, and for an
+ * out that overlaps k_new or v_new. */
 int pdk_decode_attn_append(const uint16_t* q, const uint16_t* k_new,
                            const uint16_t* v_new, uint16_t* cache_k,
                            uint16_t* cache_v, int num_blocks,

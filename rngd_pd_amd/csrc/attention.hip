@@ -38,10 +38,12 @@
 // cleared with a memset and no state survives a launch, so the kernels can be
 // captured in a HIP graph.
 
+#include <limits.h>
 #include <math.h>
 #include <stdlib.h>
 
 #include <algorithm>
+#include <functional>
 #include <mutex>
 #include <type_traits>
 
@@ -229,6 +231,26 @@ __device__ __forceinline__ void patch_v(Span& r, int span, const NewToken& nt, i
   }
 }
 
+// Streams whose tables share blocks (one request's rows at consecutive
+// positions, as a verification step sends them): in two launches each would find
+// the others' new tokens in the cache, but within one launch another workgroup
+// may not have written them yet. So each wavefront counts, one stream per lane,
+// how often the block that stream's token goes to (`written`, kNoBlock: none) is
+// among the blocks of its spans, and where one is met out of its place it goes
+// over its spans once more with those tokens taken from their rows. Where blocks
+// are each one stream's, that costs a load per workgroup and a compare per block.
+constexpr int kMaxShared = 64;   // streams whose blocks one wavefront holds
+constexpr int kNoBlock = INT_MIN;
+
+// Bit s: stream s's token goes to block id, the span's tokens from `at` on; not
+// the workgroup's own stream b at its own place, which nt covers.
+__device__ __forceinline__ uint64_t others_in_block(int written, int b, int pos, int at, int id,
+                                                    int lim, int num_blocks) {
+  const uint64_t in = __ballot(written == id);
+  if (!valid_block(id, num_blocks) || at >= lim) return 0;
+  return (pos >> 4) == (at >> 4) ? in & ~(1ull << b) : in;
+}
+
 // The read probe's stand-in for attend_span: every loaded word is folded into
 // one register, so the loads stay but no arithmetic of attention is done.
 template <int kNV>
@@ -258,15 +280,16 @@ __device__ __forceinline__ void fold_span(const Span& r, f32x4 o[8]) {
 // so the arithmetic of a query column is the same whatever columns share its
 // wavefront.
 // With kPatch (the fused RoPE path) the span's K and V take the new token nt
-// in place of the cache's contents.
-template <bool kPatch, int kNV>
+// in place of the cache's contents, after those that others(f) hands to f.
+template <bool kPatch, int kNV, class F>
 __device__ __forceinline__ void attend_span(const AttnArgs& a, Span& r, const v8 qv[4], int span,
                                             int lo, int hi, int lim, int g, int j, bool first,
                                             float& m, float& lsum, f32x4 o[8],
-                                            const NewToken& nt) {
+                                            const NewToken& nt, F others) {
   const int tv = span + 8 * g;
   const bool full = span + kSpan <= lim && valid_block(lo, a.num_blocks) &&
                     valid_block(hi, a.num_blocks);
+  others([&](const NewToken& t) { patch_k(r, span, t, g, j); });
   int blk = -1;
   if constexpr (kPatch) {
     blk = new_token_block(nt, span, lo, hi, a.num_blocks);
@@ -325,6 +348,7 @@ __device__ __forceinline__ void attend_span(const AttnArgs& a, Span& r, const v8
     }
   }
   m = m_new;
+  others([&](const NewToken& t) { patch_v<kNV>(r, span, t, g, j); });
   if constexpr (kPatch) {
     if (blk >= 0) patch_v<kNV>(r, span, nt, g, j);
   }
@@ -381,11 +405,15 @@ __device__ __forceinline__ void attend_span(const AttnArgs& a, Span& r, const v8
 // to that kernel followed by the kRope = 0 path.
 // kRope = kAppend: src is q as with 0, and the new token's k and v come as bf16
 // [B][Hkv][D] rows (k_new, v_new): into LDS, to their cache slot and into the
-// span that holds the position as with the fused RoPE. The result is that of
-// pdk_cache_append followed by the kRope = 0 path, bit for bit, without the
-// append's launch: per layer (32 query, 8 KV heads, HIP graph) B=16 ctx 512 11.0
-// -> 9.1 us, B=8 ctx 512 10.0 -> 8.4, B=16 ctx 4096 52.6 -> 50.4, B=1 ctx 8192
-// 17.3 -> 15.0, B=64 ctx 1024 (8 query heads) 51.6 -> 51.9.
+// span that holds the position as with the fused RoPE, and a span that another
+// stream's new token goes to takes that one too (others_in_block; the fused RoPE
+// path has no such streams, its caller's blocks are each one stream's). The
+// result is that of pdk_cache_append followed by the kRope = 0 path, bit for bit,
+// without the append's launch: per layer (32 query, 8 KV heads, HIP graph) B=16
+// ctx 512 11.0 -> 9.3 us, B=8 ctx 512 9.2 -> 7.5, B=16 ctx 4096 49.4 -> 47.6, B=1
+// ctx 8192 17.1 -> 14.5. (Without the look at other streams' blocks B=16 ctx 512
+// took 9.0.) Four rows of each request at consecutive positions: B=16 ctx 512
+// 8.8 -> 10.8, B=64 18.6 -> 24.6, for the spans that are gone over twice.
 // kRope = -1 is the read probe (pdk_attn_read_probe): the same launch, block
 // ids and K/V loads, none of the arithmetic, one store per thread.
 // kAct: out in the decode step's tiled activation layout (pdk::act_at, row b,
@@ -407,12 +435,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     uint16_t* ck_w, uint16_t* cv_w, const float* ssq, int n_ssq, float eps,
     const uint16_t* k_new, const uint16_t* v_new) {
   constexpr bool kRot = kRope > 0 && kRope != kAppend;   // the fused RoPE
+  constexpr bool kOthers = kRope == kAppend;
   const uint16_t* q = static_cast<const uint16_t*>(src);
   const float* part = static_cast<const float*>(src);
   __shared__ __align__(16) float sm_m[kMaxG][kMaxWaves];
   __shared__ __align__(16) float sm_l[kMaxG][kMaxWaves];
   __shared__ __align__(16) uint16_t q_rot[kRot ? kMaxG : 1][kD];   // rotated q of the group
   __shared__ __align__(16) uint16_t kv_new[2][kD];                  // rotated k, v of the new token
+  __shared__ int written_s[kOthers ? kMaxShared : 1];               // others_in_block,
+  __shared__ uint8_t slot_s[kOthers ? kMaxShared : 1];              // and the slot there
   extern __shared__ float sm_o[];                // [min(G, kMergeRows)][kORow]
 
   AttnArgs a;
@@ -530,6 +561,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     id[3] = ctab[min((sb >> 4) + 1, mb)];
   };
   const int sa0 = s_begin + wv * kSpan;
+  const int n_b = mb_b >> 16;
+  int len = 0;                                   // of stream `lane`, for written_s
+  if constexpr (kOthers) {
+    if (wv == 1 && lane < n_b) len = ctx_lens[lane];
+  }
   int id0[4];
   ids(sa0, id0);
   asm volatile("" : "+s"(ctx_raw) : "s"(id0[0]), "s"(id0[1]), "s"(id0[2]), "s"(id0[3]));
@@ -540,13 +576,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if constexpr (kRot) {
     if (ssq) rr = pdk::row_rms_load(ssq, b, n_ssq, lane);
     ifreq = inv_freq[lane];
-  }
-  // The new token's k (lanes 0-15, 8 dims each) and v (lanes 16-31), ahead of
-  // every K/V load; the other lanes repeat them.
-  v8 fresh = pdk::zero8();
-  if constexpr (kRope == kAppend) {
-    const int64_t row = ((int64_t)b * a.Hkv + h) * kD + (lane & 15) * 8;
-    fresh = pdk::ld16((lane & 16 ? v_new : k_new) + row);
   }
   const int ctx = min(ctx_raw, a.max_blocks * 16);
   const int s_end = (split == a.nsplit - 1) ? ctx : min(ctx, s_begin + a.split_tokens);
@@ -577,8 +606,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // on the other paths such a wavefront skips the loads and the spans at once.
   if constexpr (kRope > 0) first_loads();
   if constexpr (kRope == kAppend) {
-    if (wv == 0 && lane < 32)
-      *reinterpret_cast<v8*>(&kv_new[lane >> 4][(lane & 15) * 8]) = fresh;
+    // Behind the K/V loads, which nothing is to delay (both loads ahead of them
+    // in every wavefront: B=16 ctx 512 9.0 -> 9.7 us per layer): by one wavefront
+    // the new token's k (lanes 0-15, 8 dims each) and v (lanes 16-31), by another
+    // the blocks that all streams' new tokens go to (by every wavefront: 9.4).
+    if (wv == 0 && lane < 32) {
+      const int64_t row = ((int64_t)b * a.Hkv + h) * kD + (lane & 15) * 8;
+      *reinterpret_cast<v8*>(&kv_new[lane >> 4][(lane & 15) * 8]) =
+          pdk::ld16((lane & 16 ? v_new : k_new) + row);
+    }
+    if (wv == 1 && lane < n_b) {
+      const int id = tables[(int64_t)lane * a.max_blocks + min(max(len - 1, 0) >> 4, mb)];
+      const bool has = len >= 1 && len <= a.max_blocks * 16 && valid_block(id, a.num_blocks);
+      written_s[lane] = has ? id : kNoBlock;
+      slot_s[lane] = (uint8_t)((len - 1) & 15);
+    }
     __syncthreads();
   }
   if constexpr (kRot) {
@@ -652,6 +694,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   }
   const NewToken nt{pos, kv_new[0], kv_new[1] + vd0};
+  int written = kNoBlock, met = 0;
+  if constexpr (kOthers) {
+    if (lane < n_b) written = written_s[lane];
+  }
+  auto look = [&](int sa, const int* id) __attribute__((always_inline)) {
+    if constexpr (kOthers) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        met += written == (sa + (i & 1) * 16 + (i >> 1) * stride < s_end ? id[i] : -1) ? 1 : 0;
+    }
+  };
   // A wavefront's spans are sa0 + k * stride. Two of them are in registers at
   // a time (ra, rb): while one is used the other's loads are in flight, and a
   // span's registers are refilled with the span two ahead as soon as it has
@@ -659,7 +712,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   auto use = [&](auto first_c, Span& r, int s, int lo, int hi) __attribute__((always_inline)) {
     if constexpr (kRope < 0) fold_span<kNV>(r, o);
     else attend_span<(kRope > 0), kNV>(a, r, qv, s, lo, hi, s_end, g, j,
-                                       decltype(first_c)::value, m, lsum, o, nt);
+                                       decltype(first_c)::value, m, lsum, o, nt, [](auto) {});
   };
   // Spans sa and sa + stride with the span sa + 2 stride still to come: use
   // both and refill both (the second refill dead when sa + 3 stride has no
@@ -682,15 +735,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (sa0 + 2 * stride < s_end) {
       int cur[4], nxt[4];
       pair(std::true_type{}, sa0, id0, nxt);
+      look(sa0, id0);
       int sa = sa0 + 2 * stride;
       for (; sa + 2 * stride < s_end; sa += 2 * stride) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) cur[i] = nxt[i];
         pair(std::false_type{}, sa, cur, nxt);
+        look(sa, cur);
       }
       last(std::false_type{}, sa, nxt);
+      look(sa, nxt);
     } else {
       last(std::true_type{}, sa0, id0);
+      look(sa0, id0);
     }
   };
   // The fused RoPE path with whole V (kNV = 8) keeps a loop whose refills are
@@ -705,6 +762,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     use(first_c, ra0, sa, cur[0], cur[1]);
     if (sc < s_end) load_span<kNV, kVStream, knt>(a, h, sc, g, j, nxt[0], nxt[1], ra0);
     if (sb < s_end) use(std::false_type{}, rb0, sb, cur[2], cur[3]);
+    look(sa, cur);
     if (sd < s_end) load_span<kNV, kVStream, knt>(a, h, sd, g, j, nxt[2], nxt[3], rb0);
     return sc;
   };
@@ -720,6 +778,36 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int i = 0; i < 4; ++i) nxt[i] = cur[i];
         sa = pair_cond(std::false_type{}, sa, nxt, cur);
+      }
+    }
+    if constexpr (kOthers) {
+      const bool own = lane == b && pos >= s_begin && pos < s_end &&
+                       ((pos - s_begin) / kSpan) % W == wv;
+      if (__builtin_expect(__any(met > (own ? 1 : 0)), 0)) {   // once more, with others' tokens
+        m = -INFINITY;
+        lsum = 0.f;
+#pragma unroll
+        for (int n = 0; n < kNV; ++n) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int sa = sa0; sa < s_end; sa += stride) {
+          const int lo = ctab[min(sa >> 4, mb)], hi = ctab[min((sa >> 4) + 1, mb)];
+          load_span<kNV, false, false>(a, h, sa, g, j, lo, hi, ra0);
+          auto others = [&](auto f) __attribute__((always_inline)) {
+#pragma unroll 1
+            for (int half = 0; half < 2; ++half) {
+              uint64_t in = others_in_block(written, b, pos, sa + 16 * half, half ? hi : lo,
+                                            s_end, a.num_blocks);
+#pragma unroll 1
+              for (; in; in &= in - 1) {
+                const int s = __builtin_ctzll(in);
+                const int64_t row = ((int64_t)s * a.Hkv + h) * kD;
+                const int slot = __builtin_amdgcn_readfirstlane(slot_s[s]);
+                f(NewToken{sa + 16 * half + slot, k_new + row, v_new + row + vd0});
+              }
+            }
+          };
+          attend_span<true, kNV>(a, ra0, qv, sa, lo, hi, s_end, g, j, false, m, lsum, o, nt, others);
+        }
       }
     }
   }
@@ -1112,11 +1200,22 @@ extern "C" int pdk_decode_attn_append(const uint16_t* q, const uint16_t* k_new,
   pdk::clear_error();
   PDK_REQUIRE(q && k_new && v_new, "null pointer argument");
   PDK_REQUIRE(pdk::aligned16(k_new) && pdk::aligned16(v_new), "k_new/v_new must be 16-byte aligned");
-  // With several rounds of workgroups that read next to nothing each, every
-  // round's wait for the new rows costs more than the append's launch: B=64, 8
-  // KV heads, ctx 64 11.6 us per layer in two launches, 12.6 in one; ctx 256 20.6
-  // and 18.8.
-  if ((int64_t)B * n_kv_heads > kTargetWorkgroups && max_ctx <= 128) {
+  // With several rounds of workgroups, each round's wait for the new rows costs
+  // more than the append's launch where it reads next to nothing, and again
+  // where the launch is a small part of the whole (us per layer in two launches
+  // and in one, 8 KV heads: B=64 ctx 64 11.6 and 12.6, 192 17.3 and 16.7, 512 31.0
+  // and 29.8, 900 46.4 and 47.3, 2048 92.7 and 90.5; B=56 ctx 700 34.7 and 35.2,
+  // 1500 60.8 and 62.1; B=40 ctx 700 30.2 and 29.1, 1500 52.6 and 52.3). More
+  // streams than a wavefront has lanes, and rows that the output overwrites (the
+  // append has read them before the attention writes), take two launches as well.
+  const int64_t row = (int64_t)n_kv_heads * head_dim, pairs = (int64_t)B * n_kv_heads;
+  auto overwritten = [&](const uint16_t* rows) {
+    return std::less<const uint16_t*>()(rows, out + (int64_t)B * n_q_heads * head_dim) &&
+           std::less<const uint16_t*>()(out, rows + B * row);
+  };
+  const bool rounds = pairs > kTargetWorkgroups &&
+                      (max_ctx <= 128 || (pairs > 352 && max_ctx > 640 && max_ctx <= 1536));
+  if (B > kMaxShared || rounds || overwritten(k_new) || overwritten(v_new)) {
     if (int rc = pdk_cache_append(k_new, v_new, cache_k, cache_v, num_blocks, block_tables,
                                   max_blocks, ctx_lens, B, n_kv_heads, head_dim, stream))
       return rc;

@@ -66,7 +66,8 @@ class BatchDecodeAttention:
         return self._tables, ctx, max(pos) + 1
 
     def layer_attention(self, layer, q, k_new, v_new, tables, ctx, max_ctx, out=None, stream=None):
-        """One layer: write the new token's k/v at slot pos, attend over 0..pos.
+        """One layer: write the new tokens' k/v at slots pos, then attend over 0..pos
+        (streams may share blocks: each sees the others' new tokens in them).
         q [B, Hq, D], k_new/v_new [B, Hkv, D] bf16 on the device."""
         ck, cv = self.cache.k[layer], self.cache.v[layer]
         need = _attn.workspace_bytes(q.shape[0], self.Hq, max_ctx, self.cache.head_dim)

@@ -95,8 +95,9 @@ def decode_attention(q, cache_k, cache_v, block_tables, ctx_lens, max_ctx, scale
 def decode_attention_append(q, k_new, v_new, cache_k, cache_v, block_tables, ctx_lens, max_ctx,
                             scale=1.0, out=None, workspace=None, stream=None):
     """cache_append(k_new, v_new) then decode_attention, in one launch where the
-    kernel takes it (head_dim 128, 16-byte aligned rows), with the same results
-    bit for bit. k_new, v_new bf16 [B, Hkv, D]."""
+    kernel takes it (head_dim 128, 16-byte aligned rows, up to 64 streams), with
+    the same results bit for bit, also where streams' tables share the blocks
+    that the new tokens go to. k_new, v_new bf16 [B, Hkv, D]."""
     _need(k_new, "k_new")
     _need(v_new, "v_new")
     nb, H, D = _check_layer_cache(cache_k, cache_v)
