@@ -536,8 +536,8 @@ int pdk_linear_ssq_xt(const uint16_t* x, const uint16_t* wt, int B, int K, int N
 /* pdk_linear_ssq_xt's result, bit for bit, with a workspace that lets it split
  * K over workgroups: pdk_linear_ssq_ws_bytes(B, K, N) bytes (0: none needed),
  * 16-byte aligned, zeroed once before its first use and used by one stream at
- * a time; the call leaves its counters zero again. A workspace made for a
- * larger B serves a smaller one. */
+ * a time; the call leaves its counters zero again. One workspace serves calls
+ * of any shapes whose bytes it holds. */
 int64_t pdk_linear_ssq_ws_bytes(int B, int K, int N);
 int pdk_linear_ssq_ws_xt(const uint16_t* x, const uint16_t* wt, int B, int K,
                          int N, const uint16_t* residual, uint16_t* y,

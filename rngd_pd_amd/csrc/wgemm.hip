@@ -828,7 +828,7 @@ extern "C" int pdk_linear_ssq_xt(const uint16_t* x, const uint16_t* wt, int B, i
 
 extern "C" int64_t pdk_linear_ssq_ws_bytes(int B, int K, int N) {
   if (B < 1 || B > 64 || N < 1 || !wide_ssq(B, K, N)) return 0;
-  return (int64_t)kWideSplits * B * N * 4 + (int64_t)((N + 63) / 64) * 4;
+  return (int64_t)kWideCounters * 4 + (int64_t)kWideSplits * B * N * 4;
 }
 
 extern "C" int pdk_linear_ssq_ws_xt(const uint16_t* x, const uint16_t* wt, int B, int K, int N,
@@ -843,9 +843,10 @@ extern "C" int pdk_linear_ssq_ws_xt(const uint16_t* x, const uint16_t* wt, int B
   PDK_REQUIRE(workspace && workspace_bytes >= need && pdk::aligned16(workspace),
               "workspace of %lld bytes needed (got %lld)", (long long)need,
               (long long)workspace_bytes);
-  // The counters come first: their place then does not depend on B.
+  // The counters come first, as many for every shape: no call's partial sums
+  // then lie where another's counters do.
   int* counters = static_cast<int*>(workspace);
-  float* part = reinterpret_cast<float*>(counters + (N + 63) / 64);
+  float* part = reinterpret_cast<float*>(counters + kWideCounters);
   return launch_wide_ssq(x, wt, B, K, N, residual, y, ssq, part, counters, pdk::as_stream(stream));
 }
 

@@ -85,8 +85,9 @@ int launch_wide_swiglu(const uint16_t* x, const uint16_t* w, int B, int K, int M
                        float eps, uint16_t* y, hipStream_t st);
 int launch_wide_argmax(const uint16_t* x, const uint16_t* w, int B, int K, int N, const float* ssq,
                        float eps, uint16_t* logits, uint64_t* keys, hipStream_t st);
-// part: kWideSplits * B * N floats; counters: ceil(N / 64) zeros, left zero.
-constexpr int kWideSplits = 4;
+// part: kWideSplits * B * N floats; counters: ceil(N / 64) of kWideCounters
+// zeros, left zero.
+constexpr int kWideSplits = 4, kWideCounters = 4096;
 int launch_wide_ssq(const uint16_t* x, const uint16_t* w, int B, int K, int N, const uint16_t* r,
                     uint16_t* y, float* ssq, float* part, int* counters, hipStream_t st);
 

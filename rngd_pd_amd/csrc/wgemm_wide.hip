@@ -321,7 +321,8 @@ bool wide_argmax(int B, int K, int N) { return fits(B, K) && (N + 63) / 64 >= 19
 // Each class needs enough steps to pay for the partial sums (8 and more; with
 // 4 it is slower, above), and the 4 x N / 64 workgroups have to fill the chip.
 bool wide_ssq(int B, int K, int N) {
-  return fits(B, K) && K / kStepK >= 64 && N >= 4096 && N % kStepK == 0;
+  return fits(B, K) && K / kStepK >= 64 && N >= 4096 && N % kStepK == 0 &&
+         N <= 64 * kWideCounters;
 }
 
 int launch_wide_swiglu(const uint16_t* x, const uint16_t* w, int B, int K, int M, const float* ssq,

@@ -62,6 +62,27 @@ def test_argmax(cuda, B, K, N):
         assert _eq(logits, outs[0][0]) and torch.equal(tok, outs[0][1])
 
 
+def test_one_workspace_for_several_shapes(cuda):
+    """Calls of several widths in turn on one workspace, zeroed once."""
+    from rngd_pd_amd import kernels as K_
+    lib, K, shapes = _lib.lib(), 8192, [(64, 4096), (17, 4224), (33, 8192), (20, 4224)]
+    ws = torch.zeros(max(lib.pdk_linear_ssq_ws_bytes(B, K, N) for B, N in shapes) // 4,
+                     dtype=torch.int32, device=cuda)
+    for B, N in shapes + shapes[::-1]:
+        x, wt, _ = _operands(cuda, B, K, N)
+        r = to_dev(rand_bf16(np.random.default_rng(N), (B, N), 4.0))
+        print(f"shared workspace B={B} N={N}", flush=True)
+        ref, ssq_ref = r.clone(), torch.zeros((B, N // 16), dtype=torch.float32, device=cuda)
+        _lib.call("pdk_linear_ssq_tiled", x.data_ptr(), wt.data_ptr(), B, K, N, ref.data_ptr(),
+                  ref.data_ptr(), ssq_ref.data_ptr(), 0)
+        y = _tiled_in(r)
+        ssq = torch.full((B, N // 16), float("nan"), dtype=torch.float32, device=cuda)
+        _lib.call("pdk_linear_ssq_ws_xt", _tiled_in(x).data_ptr(), wt.data_ptr(), B, K, N,
+                  y.data_ptr(), y.data_ptr(), ssq.data_ptr(), ws.data_ptr(), ws.numel() * 4, 0)
+        torch.cuda.synchronize()
+        assert _eq(K_.act_untile(y, B, N), ref) and torch.equal(ssq, ssq_ref), (B, N)
+
+
 @pytest.mark.parametrize("B,K,N", [(17, 8192, 4096), (32, 14336, 4096), (33, 8192, 4224),
                                    (50, 14336, 4096), (64, 8192, 4096), (64, 4096, 4096),
                                    (16, 8192, 4096), (40, 8320, 4096)])
