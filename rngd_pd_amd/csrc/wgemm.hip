@@ -99,7 +99,10 @@ __global__ __launch_bounds__(kWaves * 64) void wgemm_kernel(const uint16_t* __re
   constexpr bool kArg = kEpi == kArgmax || kEpi == kArgmaxRms;
   constexpr int kPairs = kGLU ? 2 : 1;
   constexpr int kW = kPairs * kCols;                 // W tiles per step
-  constexpr int kDepth = depth_for(kTiles, kW);
+  // The lm_head's two column tiles at 33 to 48 rows: at depth 2 the lane's state
+  // takes 28 bytes of scratch beyond its 256 registers (N = 8016, K = 4096, B=40
+  // 25.1 us, at depth 1 23.1; B=33 24.2 and 22.7).
+  constexpr int kDepth = kArg && kTiles == 3 && kCols == 2 ? 1 : depth_for(kTiles, kW);
   __shared__ float red[kWaves][kW][256];
   __shared__ float rms[kRowScale ? 64 : 1];
   __shared__ int is_last;
@@ -485,7 +488,8 @@ int launch(const uint16_t* x, const uint16_t* w, int B, int K, int N, const uint
   // / 29.0, B=50 36.7 / 26.7 / 29.5 / -; N = 16032 B=1 32.9 / 29.0 / 26.2 / 32.9,
   // B=16 36.8 / 31.6 / 28.8 / 34.6, B=50 65.2 / 44.7 / 36.6 / -; N = 32064 B=1
   // 54.8 / 53.7 / 49.6 / 49.1, B=16 63.2 / 56.6 / 52.9 / 48.8; N = 128256 B=16
-  // 215 / 194 / 178 / 174, B=20 308 / 222 / 195 / 213. So the widest that leaves
+  // 215 / 194 / 178 / 174, B=20 308 / 222 / 195 / 213; N = 8016 B=40 30.9 / 23.1 / -
+  // / -, N = 6160 30.1 / 21.8, N = 11008 42.1 / 36.0. So the widest that leaves
   // about 200 workgroups, except that one tile is best for a few rows, and 8
   // tiles only up to 16 rows (more rows leave no registers).
   if constexpr (kAct && kEpi == kArgmaxRms) {
@@ -504,7 +508,8 @@ int launch(const uint16_t* x, const uint16_t* w, int B, int K, int N, const uint
   }
   // Wide SwiGLU tiles hold 8 weight tiles per step in registers: beyond 32
   // streams they would spill, and fewer tiles are used instead. The lm_head with
-  // tiled weights runs 4 tiles wide at every B (B = 4: 181 -> 178 us).
+  // tiled weights and row-major activations runs 4 tiles wide at every B from 1024
+  // such workgroups on (N = 128256, B = 4: 181 -> 178 us).
   constexpr bool kGLU = kEpi == kSwiGLU || kEpi == kSwiGLURms;
   const bool four = kGLU ? (wide >= 192 && B <= 32) : ((B > 8 || kTiled) && wide >= 1024);
   if (four) return launch_cols<4, kEpi, kTiled, kAct>(x, w, B, K, N, r, y, keys, st, nullptr, 1,

@@ -31,5 +31,11 @@ def test_scratch_guard_flags_only_listed_kernels():
     assert "decode_attn_kernel" in bad[0][0] and bad[0][1] == 52
 
 
+def test_scratch_guard_flags_the_lm_head_of_33_to_48_streams():
+    name = "_ZN12_GLOBAL__N_112wgemm_kernelILi3ELi2ELi8ELb1ELb1EEEvPKt"
+    assert build.scratch_kernels({name: {"ScratchSize [bytes/lane]": "28"}}) == [(name, 28)]
+    assert not build.scratch_kernels({name: {"ScratchSize [bytes/lane]": "0"}})
+
+
 def test_build_command_asks_for_the_report():
     assert "-Rpass-analysis=kernel-resource-usage" in build.hipcc_command("/tmp/x.so")

@@ -43,7 +43,8 @@ def test_swiglu(cuda, B, K, M):
 
 @pytest.mark.parametrize("B,K,N", [(17, 2048, 12225), (33, 4096, 16032), (48, 2048, 12288),
                                    (64, 2048, 20001), (64, 1152, 12288), (20, 2048, 8016),
-                                   (8, 2048, 8016), (16, 2048, 16032), (7, 2048, 6100)])
+                                   (8, 2048, 8016), (16, 2048, 16032), (7, 2048, 6100),
+                                   (33, 2048, 6160), (40, 4096, 8016), (48, 1152, 12225)])
 def test_argmax(cuda, B, K, N):
     x, wt, ssq = _operands(cuda, B, K, N)
     print(f"wide argmax B={B} K={K} N={N}", flush=True)
