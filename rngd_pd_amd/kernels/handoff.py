@@ -22,13 +22,18 @@ from .._lib import PackReq, ScatterReq, PDK_MAX_BATCH, PDK_BLOCK_SIZE
 BF16 = torch.bfloat16
 
 
+# The current stream's handle without a Stream object, which costs the host 2 us;
+# None where this torch has no such function.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+
+
 def stream_handle(stream=None):
     """hipStream_t of a torch stream (default: the current stream) as an int."""
     if stream is None:
-        if not torch.cuda.is_initialized():
+        if _raw_stream is None or not torch.cuda.is_initialized():
             return torch.cuda.current_stream().cuda_stream
-        # The same handle without a Stream object, which costs the host 2 us.
-        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        return _raw_stream(_current_device())
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
