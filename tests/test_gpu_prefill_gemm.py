@@ -133,6 +133,33 @@ def test_argmax_of_partials(cuda, N, splits):
         assert got == int(torch.argmax(total.to(BF16).float().cpu())), case
 
 
+@pytest.mark.parametrize("K,N", [(4096, 128256), (4096, 1028), (14336, 260), (256, 300),
+                                 (4096, 1027), (320, 5000)])
+def test_greedy_token(cuda, K, N):
+    """The head's token where it is clear: one row of the head along the hidden
+    state, anywhere in the vocabulary, and two equal ones (the first counts)."""
+    from rngd_pd_amd.engines.llama_decode import LlamaConfig, LlamaWeights
+    from rngd_pd_amd.engines.llama_prefill import LlamaPrefill, _Projections
+    cfg = LlamaConfig(hidden=256, n_heads=2, n_kv_heads=1, head_dim=128, inter=256, vocab=64,
+                      n_layers=1)
+    pre = LlamaPrefill(LlamaWeights.random(cfg, seed=5, device=cuda))
+    proj = _Projections(cfg, 1, pre.device)
+    print(f"greedy K={K} N={N} splits={_lib.lib().pdk_prefill_gemm_splits(1, K, N)}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(N)
+    last = torch.randn((1, K), generator=g, device=cuda).to(BF16)
+    head = (torch.randn((N, K), generator=g, device=cuda) * 0.02).to(BF16)
+    # The other logits are N(0, 0.02 sqrt(K)); the row's own is 0.2 K, at least
+    # 160 of their deviations.
+    for row in sorted({0, 3, N // 2, min(1023, N - 2), min(1024, N - 1), N - 1}):
+        kept = head[row].clone(), head[N - 1].clone()
+        head[row] = last[0] * 0.2
+        assert pre._greedy(last, head, proj) == row
+        head[N - 1] = head[row]
+        assert pre._greedy(last, head, proj) == row
+        head[N - 1] = kept[1]
+        head[row] = kept[0]
+
+
 def test_forward_on_both_sides_of_the_switches(cuda):
     """A prompt's first tokens have the same KV whatever kernels its length
     takes, and a weight the kernels cannot read takes the library."""
