@@ -40,23 +40,23 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_kernel(uint16_t* x, const vo
                                                            int splits, int64_t split_stride,
                                                            const uint16_t* w, float eps, int H,
                                                            uint16_t* out) {
-  constexpr int kNormThreads = kThreads, kNormChunks = 1024 / kThreads;  // 8 elements per chunk
+  constexpr int kChunks = kNormMaxH / 8 / kThreads;    // of 8 elements, per thread
   constexpr int kFlight = kThreads > 256 ? 8 : 2;
-  __shared__ float part[kNormThreads / 64];
+  __shared__ float part[kThreads / 64];
   const int64_t row = (int64_t)blockIdx.x * H;
   const int n8 = H >> 3;
-  v8 keep[kNormChunks], gain[kNormChunks];
+  v8 keep[kChunks], gain[kChunks];
   float ss = 0.f;
   // The weights are loaded with the row, before the reduction, so the second
   // pass waits on no memory.
 #pragma unroll
-  for (int j = 0; j < kNormChunks; ++j) {
-    const int c = threadIdx.x + j * kNormThreads;
+  for (int j = 0; j < kChunks; ++j) {
+    const int c = threadIdx.x + j * kThreads;
     gain[j] = c < n8 ? pdk::ld16(w + 8 * c) : pdk::zero8();
   }
 #pragma unroll
-  for (int j = 0; j < kNormChunks; ++j) {
-    const int c = threadIdx.x + j * kNormThreads;
+  for (int j = 0; j < kChunks; ++j) {
+    const int c = threadIdx.x + j * kThreads;
     keep[j] = pdk::zero8();
     if (c < n8) {
       v8 a = pdk::ld16(x + row + 8 * c);
@@ -109,11 +109,11 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_kernel(uint16_t* x, const vo
   __syncthreads();
   float tot = 0.f;
 #pragma unroll
-  for (int i = 0; i < kNormThreads / 64; ++i) tot += part[i];
+  for (int i = 0; i < kThreads / 64; ++i) tot += part[i];
   const float r = rsqrtf(tot / (float)H + eps);
 #pragma unroll
-  for (int j = 0; j < kNormChunks; ++j) {
-    const int c = threadIdx.x + j * kNormThreads;
+  for (int j = 0; j < kChunks; ++j) {
+    const int c = threadIdx.x + j * kThreads;
     if (c < n8) {
       const v8 a = keep[j];
       const v8 g = gain[j];

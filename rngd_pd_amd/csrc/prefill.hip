@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(uint16_t* qkv, const float
                                                       uint16_t* k_out, int64_t k_ld,
                                                       uint16_t* v_out, int64_t v_ld, uint16_t* kt,
                                                       uint16_t* vt) {
-  constexpr int kRopeHeads = kPart ? 1 : ::kRopeHeads;
+  constexpr int kHeads = kPart ? 1 : kRopeHeads;
   __shared__ uint16_t vs[kTile][kVRow];
   const int tile = blockIdx.x, n_tiles = gridDim.x;
   const int r = threadIdx.x >> 3, o = threadIdx.x & 7;
@@ -129,10 +129,10 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(uint16_t* qkv, const float
   }
   const int n_heads = NH + 2 * NKV;
   uint16_t* row = qkv + (int64_t)tc * (kPart ? NH : n_heads) * kD + 8 * o;
-  const int h0 = blockIdx.y * kRopeHeads;
-  v8 a[kRopeHeads], b[kRopeHeads];
+  const int h0 = blockIdx.y * kHeads;
+  v8 a[kHeads], b[kHeads];
 #pragma unroll
-  for (int i = 0; i < kRopeHeads; ++i) {
+  for (int i = 0; i < kHeads; ++i) {
     const int hd = min(h0 + i, n_heads - 1);
     if constexpr (kPart) {
       const float* p = part + ((int64_t)tc * n_heads + hd) * kD + 8 * o;
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(uint16_t* qkv, const float
     }
   }
 #pragma unroll
-  for (int i = 0; i < kRopeHeads; ++i) {
+  for (int i = 0; i < kHeads; ++i) {
     const int hd = h0 + i;
     if (hd >= n_heads) break;                      // uniform
     if (hd < NH + NKV) {

@@ -219,9 +219,9 @@ __global__ __launch_bounds__(256) void prefill_argmax_kernel(const float* part, 
 }
 
 // Tiles by the number of tokens. At most 64 of them leave the kernel bound by
-// W, where 128 weight rows x 4 stages (64 KiB) per CU are in flight and more
-// rows of X would only take LDS; from 129 on two token tiles share each part of
-// W. Without a K split (gate|up) the 64-column tiles of 17 to 32 tokens make a
+// W, where 128 weight rows x 3 stages (48 KiB; 64 KiB of LDS) per CU are in flight
+// and more rows of X would only take LDS; from 129 on two token tiles share each
+// part of W. Without a K split (gate|up) the 64-column tiles of 17 to 32 tokens make a
 // nearly empty second wave: 51.3 us at 17 tokens in the model, 64 x 128 tiles
 // take 42.7.
 // Splits fill 256 CUs (two workgroups each for the 36 KiB tiles), at most 8
@@ -251,6 +251,18 @@ int64_t tiles_of(const Plan& p, int T, int cols) {
 // the chip idle (at most 64 tiles of 128 x 256 here: N = 4096 and less). At 470
 // tokens: O 28.7 library, 24.1 here, down 93.0 and 64.3; but q|k|v 33.4 and 36.5,
 // gate|up 104 (with SwiGLU 115) and 120 of the best tile, 132 of these.
+// Around the second token tile (us with the kernel that reads the result,
+// library -> here):
+//   tokens   112          128          129          160          192          256
+//   q|k|v    27.2 -> 20.7 28.7 -> 21.5 41.4 -> 27.5 31.5 -> 27.8 37.1 -> 28.7 43.6 -> 29.2
+//   O        19.8 -> 15.2 27.9 -> 16.1 25.3 -> 23.0 30.3 -> 22.9 36.2 -> 23.7 26.2 -> 25.4
+//   down     53.6 -> 32.5 78.7 -> 33.6 57.3 -> 42.9 86.9 -> 43.8  106 -> 44.8 65.1 -> 46.9
+//   gate|up  59.4 -> 49.7 56.9 -> 51.3 60.3 -> 72.4 61.4 -> 74.0 66.3 -> 73.3 73.0 -> 76.5
+// From 129 tokens on gate|up by itself is slower here, in the model by less: a
+// prefill of 4 layers takes 767 us with it and 751 with the library's at 129
+// tokens, 783 and 765 at 160, 811 and 831 at 200, 847 and 866 at 256. It stays the
+// kernel's over the whole range because its sums are 32-bit up to SwiGLU's result:
+// the error of the KV against 64 bits is 0.0072 instead of 0.0078.
 bool takes(int T, int K, int rows) {
   if (T < 1 || K < 4 * kBK || K % kBK || rows < 4 || rows % 4) return false;
   return T <= 256 || (T <= 512 && tiles_of(plan_for(T, K, rows, false), T, rows) <= 64);

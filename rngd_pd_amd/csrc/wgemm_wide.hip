@@ -18,7 +18,8 @@
 //
 // Sums follow wg::sum_classes, so the results are bit for bit those of
 // wgemm_kernel. K / 128 must be a multiple of 16: 8 classes of an even number
-// of steps (two steps per loop turn, whose LDS buffers alternate).
+// of steps (two steps per loop turn, whose LDS buffers alternate). Widths such as
+// 3072, 5120, 11008 and 13824 are not, and their products keep wgemm_kernel.
 //
 // Measured (us, launches of a HIP graph over weights that do not fit the last-
 // level cache, before -> after): gate|up M = 14336, K = 4096 B=50 66.9 -> 44.5,
